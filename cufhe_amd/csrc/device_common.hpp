@@ -62,30 +62,36 @@ template <class TP>
 inline constexpr uint32_t kMaskRound = 1u << (32 - 2 - TP::nbit);
 
 // Double (already scaled to torus units * 2^w) to a Torus32/Torus64 word,
-// rounding to nearest and wrapping modulo 2^w (reference uses llrint for
-// Torus32 and include/utils_gpu.cuh:48-65 for Torus64).
+// rounding to nearest even and wrapping modulo 2^w (reference uses llrint for
+// Torus32 and include/utils_gpu.cuh:48-65 for Torus64). Both widths peel
+// multiples of 2^32 off with exact FMAs and read the integer out of the
+// mantissa: adding 1.5 * 2^52 rounds at the unit position, so the low words
+// of the sum are the integer's. The Torus64 form takes 10 instructions; a
+// 64-bit integer conversion with its range test and mantissa shift took about
+// 40, which a lone lvl2 wave cannot hide (1000 lvl2 annihilations 466 -> 410 us,
+// one lvl02 MUX gate 21.7 -> 20.1 ms; the 2048-gate mix waits for its key
+// loads instead, 50.2 ms either way).
 template <class T>
-__device__ __forceinline__ T double_to_torus(double v)
+__host__ __device__ __forceinline__ T double_to_torus(double v)
 {
+    constexpr double two32 = 4294967296.0, unit = 6755399441055744.0;  // 2^32, 1.5 * 2^52
+    auto bits = [](double t) { return static_cast<uint64_t>(__builtin_bit_cast(uint64_t, t)); };
     if constexpr (sizeof(T) == 4) {
-        // rint(v) mod 2^32 in four instructions: q = rint(v / 2^32) and
-        // r = v - q 2^32 (exact: |r| <= 2^31, a multiple of v's ulp), then
-        // the low word of r + 1.5 * 2^52 is rint(r) mod 2^32 (round to nearest
-        // even at the unit position; |r| < 2^51). rint(v) = q 2^32 + rint(r)
-        // with q 2^32 even, so the result equals (uint32_t)(int64_t)rint(v).
-        const double q = rint(v * (1.0 / 4294967296.0));
-        const double r = fma(-q, 4294967296.0, v);
-        const double t = r + 6755399441055744.0;
-        return static_cast<T>(static_cast<uint64_t>(__double_as_longlong(t)));
+        // v = q 2^32 + r exactly (|r| <= 2^31, a multiple of v's ulp), and
+        // q 2^32 is even, so rint(v) = q 2^32 + rint(r)
+        const double q = __builtin_rint(v * (1.0 / two32));
+        const double r = __builtin_fma(-q, two32, v);
+        return static_cast<T>(bits(r + unit));
     }
     else {
-        const double r = rint(v);
-        if (fabs(r) < 9223372036854775808.0) return static_cast<T>(static_cast<int64_t>(r));
-        const uint64_t bits = static_cast<uint64_t>(__double_as_longlong(r));
-        const int ex = static_cast<int>((bits >> 52) & 0x7FF) - 1075;
-        const uint64_t m = (bits & 0x000FFFFFFFFFFFFFULL) | 0x0010000000000000ULL;
-        const uint64_t mag = ex >= 64 ? 0 : (m << ex);  // ex >= 11 here
-        return (bits >> 63) ? static_cast<T>(0 - mag) : static_cast<T>(mag);
+        // v = q 2^64 + h 2^32 + l exactly with |h| <= 2^31, |l| <= 2^31
+        const double q = __builtin_rint(v * (1.0 / (two32 * two32)));
+        const double r = __builtin_fma(-q, two32 * two32, v);
+        const double h = __builtin_rint(r * (1.0 / two32));
+        const double l = __builtin_fma(-h, two32, r);
+        // rint(l) + 2^51 and h: the sum of the mantissas modulo 2^64
+        const uint64_t lo = bits(l + unit) - bits(unit);
+        return static_cast<T>(lo + (bits(h + unit) << 32));
     }
 }
 
