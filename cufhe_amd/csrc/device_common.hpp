@@ -95,6 +95,15 @@ __host__ __device__ __forceinline__ T double_to_torus(double v)
     }
 }
 
+// The same for a Torus32 value given in turns (units of 2^32): the fraction
+// v - rint(v) is exact.
+__host__ __device__ __forceinline__ uint32_t turns_to_torus32(double v)
+{
+    const double r = v - __builtin_rint(v);
+    return static_cast<uint32_t>(
+        __builtin_bit_cast(uint64_t, __builtin_fma(r, 4294967296.0, 6755399441055744.0)));
+}
+
 template <class T>
 inline constexpr double kTorusScale = sizeof(T) == 4 ? 4294967296.0 : 18446744073709551616.0;
 
@@ -129,15 +138,6 @@ inline int device_cu_count()
         __atomic_store_n(&cached[dev], v, __ATOMIC_RELAXED);
     }
     return v;
-}
-
-// Grid for workgroups of up to c jobs with the jobs spread evenly: the fewest
-// whole waves of CUs that hold njobs (never more workgroups than jobs).
-inline int spread_grid(int njobs, int c)
-{
-    const int cus = device_cu_count();
-    const int rounds = (njobs + c * cus - 1) / (c * cus);
-    return njobs < rounds * cus ? njobs : rounds * cus;
 }
 
 // One key-switch job: out_lvl0 = KS(ca*in0 + cb*in1 (+offset on b)).

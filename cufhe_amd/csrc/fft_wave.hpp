@@ -219,6 +219,7 @@ struct FFTTables {
     const cplx* tw64;
     const cplx* cr;
     const cplx* tws;  // tws[l] = exp(-2*pi*i*l/H)
+    const cplx* roots = nullptr;  // N = 1024: fft512.hpp's tables
 };
 
 // Twiddle sequences computed from one or two table entries by repeated
@@ -277,11 +278,10 @@ __device__ __forceinline__ int slot_t2(int row, int c, int x)
         return fft_t2<LAY == 1>(row, c, x ^ c);
 }
 
+// (fwd_a behind its products with cr)
 template <int R>
-__device__ __forceinline__ void fwd_a(cplx (&x)[R], const FFTTables& tb, int lane)
+__device__ __forceinline__ void fwd_a_dft(cplx (&x)[R], const FFTTables& tb, int lane)
 {
-#pragma unroll
-    for (int r = 1; r < R; r++) x[r] = cmul(x[r], tb.cr[r]);
     dft_reg<R, false>(x);
     TwiddleSeq ts = stage_a_twiddles(tb, lane);
 #pragma unroll
@@ -289,6 +289,13 @@ __device__ __forceinline__ void fwd_a(cplx (&x)[R], const FFTTables& tb, int lan
         x[k2] = cmul(x[k2], ts.t);
         if (k2 + 1 < R) ts.next();
     }
+}
+template <int R>
+__device__ __forceinline__ void fwd_a(cplx (&x)[R], const FFTTables& tb, int lane)
+{
+#pragma unroll
+    for (int r = 1; r < R; r++) x[r] = cmul(x[r], tb.cr[r]);
+    fwd_a_dft<R>(x, tb, lane);
 }
 // fwd_a of two transforms with each twiddle read once
 template <int R>
@@ -418,8 +425,9 @@ __device__ __forceinline__ void t1_load_inv(cplx (&x)[R], const cplx* lds, int l
 #pragma unroll
     for (int k2 = 0; k2 < R; k2++) x[k2] = lds_load(&lds[slot_t1<LAY>(k2, lane)]);
 }
+// (inv_c before its products with cr)
 template <int R>
-__device__ __forceinline__ void inv_c(cplx (&x)[R], const FFTTables& tb, int lane)
+__device__ __forceinline__ void inv_c_dft(cplx (&x)[R], const FFTTables& tb, int lane)
 {
     {
         TwiddleSeq ts = stage_a_twiddles(tb, lane);
@@ -430,6 +438,11 @@ __device__ __forceinline__ void inv_c(cplx (&x)[R], const FFTTables& tb, int lan
         }
     }
     dft_reg<R, true>(x);
+}
+template <int R>
+__device__ __forceinline__ void inv_c(cplx (&x)[R], const FFTTables& tb, int lane)
+{
+    inv_c_dft<R>(x, tb, lane);
 #pragma unroll
     for (int r = 1; r < R; r++) x[r] = cmulc(x[r], tb.cr[r]);
 }

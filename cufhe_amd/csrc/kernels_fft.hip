@@ -1,8 +1,8 @@
 // FFT-backend kernels: key conversion, batched blind rotation, plain
 // per-gate kernels, key switching, MUX combine, and FFNT entry points.
 #include "br_fft.hpp"
-#include "br_fft_kbs.hpp"
 #include "br_fft_kbw.hpp"
+#include "br_fft_pw.hpp"
 #include "keyswitch.hpp"
 #include "launch.hpp"
 
@@ -158,118 +158,41 @@ static int br_fft_resident_groups()
 }
 
 // ---------------------------------------------------------------------------
-// Batched key-bundle rotation at lvl1 with the key shared by the workgroup's
-// C jobs through an LDS ring (br_fft_kbs.hpp). One workgroup of 2C waves per
-// CU (C = 6: 12 waves, 138 KiB LDS).
-template <int C>
-__global__ __launch_bounds__(128 * C, 1) void k_br_fft_kbs(const BrJob* __restrict__ jobs,
-                                                            int njobs, uint32_t mu,
-                                                            FourierKeys<lvl1param> K)
+// Batched key-bundle rotation, one wave per digit polynomial (br_fft_pw.hpp):
+// S::J jobs per workgroup; the workgroups walk the job groups with a grid
+// stride.
+template <class S, int WPE>
+__global__ __launch_bounds__(S::NT, WPE) void k_br_fft_pw(const BrJob* __restrict__ jobs, int njobs,
+                                                          typename S::T mu,
+                                                          FourierKeys<typename S::P> K)
 {
-    using P = lvl1param;
-    constexpr int N = P::n, H = N / 2, R = H / 64, n0 = lvl0param::n;
-    constexpr int NT = 128 * C;
-    __shared__ KbsShared<C> sm;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int slot = wave >> 1, j = wave & 1;
-    const int t = threadIdx.x;
-    for (int i = t; i < 64; i += NT) {
-        sm.twl[i] = K.fft.twl[i];
-        sm.tws[i] = K.fft.tws[i];
-    }
-    for (int i = t; i < 64; i += NT) {
-        sm.tw64[i] = K.fft.tw64[i];
-        sm.e2n_lo[i] = K.e2n[i];
-    }
-    for (int i = t; i < R; i += NT) sm.cr[i] = K.fft.cr[i];
-    for (int i = t; i < 2 * N / 64; i += NT) sm.e2n_hi[i] = K.e2n[64 * i];
-    const int raw = blockIdx.x * C + slot;
-    const bool live = raw < njobs;
-    const BrJob jb = jobs[live ? raw : njobs - 1];
+    using P = typename S::P;
+    using T = typename S::T;
+    constexpr int n0 = lvl0param::n;
     constexpr uint32_t rnd = kMaskRound<P>;
-    for (int i = t & 127; i <= n0; i += 128) {
-        uint32_t v = static_cast<uint32_t>(jb.ca) * jb.in0[i];
-        if (jb.in1) v += static_cast<uint32_t>(jb.cb) * jb.in1[i];
-        if (i < n0)
-            sm.abar[slot][i] = static_cast<uint16_t>(mod_switch<P>(v + rnd));
-        else
-            sm.bar[slot] = 2 * N - mod_switch<P>(v + jb.offset);
-    }
+    __shared__ PwShared<S> sm;
+    PwWave<S> w(sm, K, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
+    w.load_tables(threadIdx.x);
     __syncthreads();
-    AccStore<P> acc;
-    blind_rotate_kbs<C>(sm, slot, j, mu, acc.reg, K.bk);
-    if (live) {
-        if (jb.flags & kBrOutTrlwe)
-            trlwe_store<P>(acc, j, static_cast<uint32_t*>(jb.out));
-        else
-            sample_extract_store<P>(acc, j, static_cast<uint32_t*>(jb.out));
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Batched key-bundle rotation at lvl1, one wave per job, key shared by the
-// workgroup's jobs through an LDS ring (br_fft_kbw.hpp). One workgroup of C
-// waves per CU (C = 8: 2 waves/SIMD, 141 KiB LDS). The launcher spreads the
-// jobs evenly over the fewest whole waves of CUs that hold them (at most C
-// per workgroup); waves without a job only stream the key, and fewer
-// rotating waves per CU finish a round sooner (one: 3.5 ms, eight: 6.3 ms).
-template <int C>
-__global__ __launch_bounds__(64 * C, 8 / C) void k_br_fft_kbw(const BrJob* __restrict__ jobs,
-                                                           int njobs, uint32_t mu,
-                                                           FourierKeys<lvl1param> K)
-{
-    using P = lvl1param;
-    constexpr int N = P::n, H = N / 2, R = H / 64, n0 = lvl0param::n;
-    constexpr int NT = 64 * C;
-    __shared__ KbwShared<C> sm;
-    const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int t = threadIdx.x;
-    for (int i = t; i < 64; i += NT) {
-        sm.twl[i] = K.fft.twl[i];
-        sm.tws[i] = K.fft.tws[i];
-    }
-    for (int i = t; i < 64; i += NT) {
-        sm.tw64[i] = K.fft.tw64[i];
-        sm.e2n_lo[i] = K.e2n[i];
-    }
-    for (int i = t; i < R; i += NT) sm.cr[i] = K.fft.cr[i];
-    for (int i = t; i < 2 * N / 64; i += NT) sm.e2n_hi[i] = K.e2n[64 * i];
-    // jobs spread evenly over the grid: workgroup b takes [b n / G, (b+1) n / G)
-    const int first = static_cast<int>((static_cast<int64_t>(blockIdx.x) * njobs) / gridDim.x);
-    const int count =
-        static_cast<int>((static_cast<int64_t>(blockIdx.x + 1) * njobs) / gridDim.x) - first;
-    const bool live = slot < count;
-    if (!live) {
-        // no job for this wave: stream its share of the key, meet the barriers
-        __syncthreads();
-        KbwKeyPipe<C> pipe(sm, slot, t & 63, K.bk);
-        pipe.run_loader_only();
-        return;
-    }
-    const BrJob jb = jobs[first + slot];
-    constexpr uint32_t rnd = kMaskRound<P>;
-    for (int i = t & 63; i <= n0; i += 64) {
-        uint32_t v = static_cast<uint32_t>(jb.ca) * jb.in0[i];
-        if (jb.in1) v += static_cast<uint32_t>(jb.cb) * jb.in1[i];
-        if (i < n0)
-            sm.abar[slot][i] = static_cast<uint16_t>(mod_switch<P>(v + rnd));
-        else
-            sm.bar[slot] = 2 * N - mod_switch<P>(v + jb.offset);
-    }
-    __syncthreads();
-    uint32_t acc[2][16];
-    blind_rotate_kbw<C>(sm, slot, mu, acc, K.bk);
-    {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            AccStore<P> a;
-#pragma unroll
-            for (int r = 0; r < 16; r++) a.reg[r] = acc[j][r];
-            if (jb.flags & kBrOutTrlwe)
-                trlwe_store<P>(a, j, static_cast<uint32_t*>(jb.out));
-            else
-                sample_extract_store<P>(a, j, static_cast<uint32_t*>(jb.out));
-        }
+    const int ngroups = (njobs + S::J - 1) / S::J;
+    for (int grp = blockIdx.x; grp < ngroups; grp += gridDim.x) {
+        const int raw = grp * S::J + w.slot;
+        const bool live = raw < njobs;
+        const BrJob jb = jobs[live ? raw : njobs - 1];
+        auto pre = [&](int i) -> uint32_t {
+            uint32_t v = static_cast<uint32_t>(jb.ca) * jb.in0[i];
+            if (jb.in1) v += static_cast<uint32_t>(jb.cb) * jb.in1[i];
+            return v;
+        };
+        auto abar = [&](int i) -> uint32_t {
+            return __builtin_amdgcn_readfirstlane(mod_switch<P>(pre(i) + rnd));
+        };
+        const uint32_t bar =
+            __builtin_amdgcn_readfirstlane(2 * S::N - mod_switch<P>(pre(n0) + jb.offset));
+        w.rotate(live, bar, mu, abar);
+        if (live && w.qi == 0)
+            pw_store<P>(reinterpret_cast<const T*>(w.buf(w.slot, w.j, 0)), w.j, w.lane,
+                        jb.flags & kBrOutTrlwe, static_cast<T*>(jb.out));
     }
 }
 
@@ -771,58 +694,92 @@ void launch_xai_poly(int32_t* out, hipStream_t st)
 template void launch_xai_poly<lvl1param>(int32_t*, hipStream_t);
 template void launch_xai_poly<lvl2param>(int32_t*, hipStream_t);
 
+// lvl1 key-bundle rotation (br_fft_pw.hpp). c = 1, 2, 4: that many jobs per
+// workgroup throughout; else (6, 8, the default) the mix that takes the fewest
+// rounds of the CUs: four jobs per CU share a key pass and the LDS best
+// (2.97 ms a round of 1024 jobs, 11.3 ms for 4096), a CU with two or one is
+// done sooner (1.78 ms for 512, 1.21 ms for 256; MI355X). So full rounds run
+// at four and what is left at the smallest width that holds it in one round.
+// Eight-wave workgroups of one wave per job, the form before, took 3.5 / 3.7 /
+// 4.2 / 12.0 ms for 256 / 512 / 1024 / 4096 jobs.
+template <int J, int DPW, int PF, int HELP>
+static void launch_pw_lvl1(const BrJob* jobs, int njobs, uint32_t mu,
+                           const FourierKeys<lvl1param>& K, hipStream_t st)
+{
+    using S = PwShape<lvl1param, J, 1, DPW, PF, HELP>;
+    if (njobs > 0)
+        hipLaunchKernelGGL((k_br_fft_pw<S, 2>), dim3((njobs + J - 1) / J), dim3(S::NT), 0, st, jobs,
+                           njobs, mu, K);
+}
+static void launch_br_kb_lvl1(const BrJob* jobs, int njobs, int c, uint32_t mu,
+                              const FourierKeys<lvl1param>& K, hipStream_t st)
+{
+    const int cus = device_cu_count();
+    int four = 0;
+    if (c == 4) {
+        four = njobs;
+    }
+    else if (c != 1 && c != 2) {
+        four = njobs / (4 * cus) * (4 * cus);
+        if (njobs - four > 2 * cus) four = njobs;
+    }
+    const int left = njobs - four;
+    launch_pw_lvl1<4, 2, 4, 0>(jobs, four, mu, K, st);
+    if (c == 2 || (c != 1 && left > cus))
+        launch_pw_lvl1<2, 1, 8, 0>(jobs + four, left, mu, K, st);
+    else
+        launch_pw_lvl1<1, 1, 8, 4>(jobs + four, left, mu, K, st);
+}
+
 template <class P, bool KB>
 void launch_br_fft(const BrJob* jobs, int njobs, int c, typename P::T mu,
                    const FourierKeys<P>& K, hipStream_t st)
 {
     if (njobs <= 0) return;
-    const dim3 block(128 * c);
-    const dim3 grid((njobs + c - 1) / c);
-    switch (c) {
-        case 1: {
-            // one resident grid (grid-stride over the jobs) for the Torus64
-            // rotation, whose key (167 MB, KB 250 MB) outgrows the caches
-            // once the workgroups drift apart
-            dim3 g1 = grid;
-            if constexpr (sizeof(typename P::T) == 8) {
-                const int cap = br_fft_resident_groups<P, KB, 1>();
-                if (cap > 0 && static_cast<int>(g1.x) > cap) g1.x = cap;
+    if constexpr (KB && sizeof(typename P::T) == 4) {
+        launch_br_kb_lvl1(jobs, njobs, c, mu, K, st);
+    }
+    else {
+        const dim3 block(128 * c);
+        const dim3 grid((njobs + c - 1) / c);
+        switch (c) {
+            case 1: {
+                // one resident grid (grid-stride over the jobs) for the Torus64
+                // rotation, whose key (167 MB, KB 250 MB) outgrows the caches
+                // once the workgroups drift apart
+                dim3 g1 = grid;
+                if constexpr (sizeof(typename P::T) == 8) {
+                    const int cap = br_fft_resident_groups<P, KB, 1>();
+                    if (cap > 0 && static_cast<int>(g1.x) > cap) g1.x = cap;
+                }
+                hipLaunchKernelGGL((k_br_fft<P, KB, 1>), g1, block, 0, st, jobs, njobs, mu, K);
+                break;
             }
-            hipLaunchKernelGGL((k_br_fft<P, KB, 1>), g1, block, 0, st, jobs, njobs, mu, K);
-            break;
-        }
-        case 2: {
-            // Torus64: two jobs (136 KiB LDS) per workgroup in a resident grid,
-            // their key loads issued together (a tuning option; one job per
-            // workgroup measured faster on the lvl02 mix)
-            dim3 g2 = grid;
-            if constexpr (sizeof(typename P::T) == 8) {
-                const int cap = br_fft_resident_groups<P, KB, 2>();
-                if (cap > 0 && static_cast<int>(g2.x) > cap) g2.x = cap;
+            case 2: {
+                // Torus64: two jobs (136 KiB LDS) per workgroup in a resident grid,
+                // their key loads issued together (a tuning option; one job per
+                // workgroup measured faster on the lvl02 mix)
+                dim3 g2 = grid;
+                if constexpr (sizeof(typename P::T) == 8) {
+                    const int cap = br_fft_resident_groups<P, KB, 2>();
+                    if (cap > 0 && static_cast<int>(g2.x) > cap) g2.x = cap;
+                }
+                hipLaunchKernelGGL((k_br_fft<P, KB, 2>), g2, block, 0, st, jobs, njobs, mu, K);
+                break;
             }
-            hipLaunchKernelGGL((k_br_fft<P, KB, 2>), g2, block, 0, st, jobs, njobs, mu, K);
-            break;
+            case 4:
+                if constexpr (sizeof(typename P::T) == 4)
+                    hipLaunchKernelGGL((k_br_fft<P, KB, 4>), grid, block, 0, st, jobs, njobs, mu,
+                                       K);
+                break;
+            case 8:
+                if constexpr (sizeof(typename P::T) == 4)
+                    hipLaunchKernelGGL((k_br_fft<P, KB, 8>), grid, block, 0, st, jobs, njobs, mu,
+                                       K);
+                break;
+            default:
+                break;
         }
-        case 4:
-            if constexpr (sizeof(typename P::T) == 4)
-                hipLaunchKernelGGL((k_br_fft<P, KB, 4>), grid, block, 0, st, jobs, njobs, mu,
-                                   K);
-            break;
-        case 8:
-            // key bundle: one wave per job (k_br_fft_kbw); otherwise two
-            if constexpr (KB && sizeof(typename P::T) == 4)
-                hipLaunchKernelGGL((k_br_fft_kbw<8>), dim3(spread_grid(njobs, 8)), dim3(64 * 8), 0,
-                                   st, jobs, njobs, mu, K);
-            else if constexpr (sizeof(typename P::T) == 4)
-                hipLaunchKernelGGL((k_br_fft<P, KB, 8>), grid, block, 0, st, jobs, njobs, mu,
-                                   K);
-            break;
-        case 6:
-            if constexpr (KB && sizeof(typename P::T) == 4)
-                hipLaunchKernelGGL((k_br_fft_kbs<6>), grid, block, 0, st, jobs, njobs, mu, K);
-            break;
-        default:
-            break;
     }
 }
 template void launch_br_fft<lvl1param, true>(const BrJob*, int, int, uint32_t,

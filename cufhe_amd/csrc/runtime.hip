@@ -19,6 +19,7 @@
 #include "br_ntt.hpp"
 #include "br_ntt64.hpp"
 #include "engine.hpp"
+#include "fft512.hpp"
 #include "ks_gemm.hpp"
 #include "launch.hpp"
 
@@ -50,6 +51,7 @@ struct TableSet {
     cplx* cr = nullptr;
     cplx* tws = nullptr;
     cplx* e2n = nullptr;
+    cplx* roots = nullptr;  // N = 1024 only
 };
 
 // NTT-backend tables (Montgomery form), see ntt_wave.hpp.
@@ -132,6 +134,27 @@ std::vector<cplx> e2n_table(int N)
     return p;
 }
 
+// fft512.hpp's root tables: per block of angle theta (the roots of X^n -
+// exp(i theta)) cos and tan of theta / 2, / 4, / 8 and / 8 + pi / 4.
+std::vector<cplx> fft512_tables()
+{
+    std::vector<cplx> t(fft512::kTabWords);
+    auto fill = [&](cplx* out, int blocks, auto n_of) {
+        for (int b = 0; b < blocks; b++) {
+            // theta = pi / (2 blocks) * (1 + 4 n): 8 blocks after three levels, 64 after six
+            const long double pi = 3.14159265358979323846264338327950288L;
+            const long double theta = pi * (1 + 4 * n_of(b)) / (2 * blocks);
+            const long double ang[4] = {theta / 2, theta / 4, theta / 8, theta / 8 + pi / 4};
+            for (int w = 0; w < 4; w++)
+                out[w * blocks + b] = cplx{static_cast<double>(cosl(ang[w])), static_cast<double>(tanl(ang[w]))};
+        }
+    };
+    auto rev3 = [](int v) { return ((v & 1) << 2) | (v & 2) | (v >> 2); };
+    fill(t.data(), 8, [&](int o) { return o; });
+    fill(t.data() + fft512::kTab1, 64, [&](int l) { return (l >> 3) + 8 * rev3(l & 7); });
+    return t;
+}
+
 template <class P>
 int build_tables(TableSet<P>& ts)
 {
@@ -159,6 +182,7 @@ int build_tables(TableSet<P>& ts)
     CUFHE_HIP_TRY(up(&ts.cr, cr));
     CUFHE_HIP_TRY(up(&ts.tws, tws));
     CUFHE_HIP_TRY(up(&ts.e2n, E));
+    if constexpr (N == 1024) CUFHE_HIP_TRY(up(&ts.roots, fft512_tables()));
     return CUFHE_OK;
 }
 
@@ -272,6 +296,7 @@ FourierKeys<P> keys_view(const TableSet<P>& ts, const cplx* bk)
     k.fft.tw64 = ts.tw64;
     k.fft.cr = ts.cr;
     k.fft.tws = ts.tws;
+    k.fft.roots = ts.roots;
     return k;
 }
 
@@ -283,6 +308,7 @@ void free_tables(TableSet<P>& ts)
     (void)hipFree(ts.cr);
     (void)hipFree(ts.tws);
     (void)hipFree(ts.e2n);
+    (void)hipFree(ts.roots);
     ts = TableSet<P>{};
 }
 
@@ -872,20 +898,16 @@ int lvl1_pick_c(int c, int nbr)
             c = 2;
         }
         else if (k.kb) {
-            // The one-wave-per-job kernel spreads the jobs over all CUs (at
-            // most 8 per workgroup; waves without a job only stream the key)
-            // and is the fastest at every batch size (MI355X, BR ms, C = 6 /
-            // 8): 256 jobs 5.84 / 3.54, 1024: 5.84 / 4.27, 1536: 6.19 / 5.55,
-            // 2048: 12.05 / 6.41, 3072: 11.73 / 11.11, 4096: 17.71 / 12.41.
+            // the mix of workgroup widths that launch_br_kb_lvl1 picks by the
+            // number of jobs
             c = 8;
         }
         else {
             c = 1;
         }
     }
-    // 6: the kernels that share key chunks among six jobs through LDS (NTT
-    // backend, all modes; FFT backend, key bundle); 8 with the key bundle:
-    // one wave per job, key shared by eight
+    // 6: the NTT kernels that share key chunks among six jobs through LDS; with
+    // the FFT key bundle 6 and 8 are the mix
     if (c == 6) return (k.backend == CUFHE_BACKEND_NTT || k.kb) ? 6 : -1;
     if (c != 1 && c != 2 && c != 4 && c != 8) return -1;
     return c;
