@@ -49,14 +49,17 @@ struct KsTraits {
 };
 
 // Key switch of the combination ca*in0 + cb*in1 (+offset on the body) for
-// one job, spread over NW waves of a workgroup (one job's key switch is a
-// long dependent gather loop over dn x t KSK rows; split NW ways its latency
-// is hidden): wave w takes the switched coefficients j in its 1/NW share,
-// each lane accumulates output columns lane + 64 c (c < 10), the partial
-// sums go through red[NW][n0 + 1] in LDS, and threads [0, 64 NW) sum them
-// into out. All lanes of a wave see the same j and digit sequence, so
-// branches are wave-uniform and each KSK row read is a coalesced run over
-// columns. Integer sums mod 2^32, so the split does not change a bit.
+// one job, spread over NW waves of a workgroup: wave w takes the switched
+// coefficients j in its 1/NW share, each lane accumulates output columns
+// lane + 64 c (c < 10), the partial sums go through red[NW][n0 + 1] in LDS,
+// and threads [0, 64 NW) sum them into out. Integer sums mod 2^32, so the
+// split does not change a bit.
+// A job reads dn x t KSK rows of 2.5 KB (18 MB at lvl1), so one CU is bound by
+// its L2 -> VGPR path, and before that by latency: the t rows of a coefficient
+// are loaded together, one coefficient ahead of their sums, and the digits of
+// 64 coefficients are prepared by the lanes and read back one by one. With each
+// row's loads next to its sums one lvl1 job took 459 us, 1024 took 627 and 4096
+// 4420; now 144, 538 and 2138 (1024 jobs: 24 TB/s out of the L2s).
 // `wave` is the wave's index within the NW waves of this job; every thread
 // of the workgroup must call it (one __syncthreads inside).
 template <class KS, bool SUBSET, int NW>
@@ -94,27 +97,69 @@ __device__ __forceinline__ void key_switch_waves(uint32_t* out, const typename K
     }
     const uint32_t j0 = first + static_cast<uint32_t>(wave) * share;
     const uint32_t j1 = j0 + share < TR::dn ? j0 + share : TR::dn;
-#pragma unroll 4
-    for (uint32_t j = j0; j < j1; j++) {
-        DT tmp = ua * in0[j] + TR::kOffset;
-        if (in1) tmp += ub * in1[j];
+    constexpr uint32_t kDigits = KS::t * KS::basebit;  // bits of all digits of a coefficient
+    static_assert(KS::basebit == 2 && kDigits <= 32, "digits in {-2, .., 1}, packed in a word");
+    struct Rows {
+        uint32_t x[KS::t][NC];
+    };
+    // the rows of a coefficient's nonzero digits
+    auto load = [&](uint32_t j, uint32_t digits) {
         const uint32_t* kj = ksk + static_cast<size_t>(j - first) * TR::coef_words;
+        Rows r;
 #pragma unroll
         for (uint32_t k = 0; k < KS::t; k++) {
-            const int32_t val =
-                static_cast<int32_t>((tmp >> (TR::W - (k + 1) * KS::basebit)) &
-                                     ((static_cast<DT>(1) << KS::basebit) - 1)) -
-                static_cast<int32_t>(TR::numbase);
-            if (val == 0) continue;
-            const uint32_t* row = kj + k * TR::digit_words + (abs(val) - 1) * TR::row_words;
+            const uint32_t v = (digits >> (kDigits - (k + 1) * KS::basebit)) & 3u;
+            if (v != 2) {
+                const uint32_t* row = kj + k * TR::digit_words + (v == 0 ? TR::row_words : 0);
 #pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const int i = lane + 64 * c;
-                if (i <= static_cast<int>(TR::n0)) {
-                    const uint32_t x = row[i];
-                    res[c] = val > 0 ? res[c] - x : res[c] + x;
+                for (int c = 0; c < NC; c++) {
+                    const int i = lane + 64 * c;
+                    r.x[k][c] = row[i <= static_cast<int>(TR::n0) ? i : static_cast<int>(TR::n0)];
                 }
             }
+        }
+        return r;
+    };
+    auto add = [&](const Rows& r, uint32_t digits) {
+#pragma unroll
+        for (uint32_t k = 0; k < KS::t; k++) {
+            const uint32_t v = (digits >> (kDigits - (k + 1) * KS::basebit)) & 3u;
+            if (v < 2) {  // digit -2 or -1
+#pragma unroll
+                for (int c = 0; c < NC; c++) res[c] += r.x[k][c];
+            }
+            else if (v == 3) {  // digit 1
+#pragma unroll
+                for (int c = 0; c < NC; c++) res[c] -= r.x[k][c];
+            }
+        }
+    };
+    for (uint32_t base = j0; base < j1; base += 64) {
+        uint32_t mine = 0;
+        const uint32_t jl = base + static_cast<uint32_t>(lane);
+        if (jl < j1) {
+            DT tmp = ua * in0[jl] + TR::kOffset;
+            if (in1) tmp += ub * in1[jl];
+            mine = static_cast<uint32_t>(tmp >> (TR::W - kDigits)) & ((1u << kDigits) - 1);
+        }
+        const uint32_t n = j1 - base < 64 ? j1 - base : 64;
+        // digits of coefficient base + i (wave-uniform); the last one again past the end
+        auto at = [&](uint32_t i) {
+            return static_cast<uint32_t>(__builtin_amdgcn_readlane(mine, i < n ? i : n - 1));
+        };
+        auto index = [&](uint32_t i) { return base + (i < n ? i : n - 1); };
+        uint32_t da = at(0), db;
+        Rows a = load(index(0), da), b;
+#pragma unroll 1
+        for (uint32_t i = 0; i < n; i += 2) {
+            db = at(i + 1);
+            b = load(index(i + 1), db);
+            asm volatile("" ::: "memory");  // the loads stay ahead of the sums
+            add(a, da);
+            da = at(i + 2);
+            a = load(index(i + 2), da);
+            asm volatile("" ::: "memory");
+            if (i + 1 < n) add(b, db);
         }
     }
 #pragma unroll
