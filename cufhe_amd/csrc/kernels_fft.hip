@@ -1,7 +1,6 @@
 // FFT-backend kernels: key conversion, batched blind rotation, plain
 // per-gate kernels, key switching, MUX combine, and FFNT entry points.
 #include "br_fft.hpp"
-#include "br_fft_kbw.hpp"
 #include "br_fft_pw.hpp"
 #include "keyswitch.hpp"
 #include "launch.hpp"
@@ -333,163 +332,115 @@ __global__ __launch_bounds__(512, 1) void k_gate_lvl1_fft(
 }
 
 // ---------------------------------------------------------------------------
-// Plain per-gate form with the key bundle at lvl1 (IKS then BR): one gate per
-// workgroup of eight waves. The gate's rotation (MUX/NMUX: two rotations) runs
-// on wave 0 (and 1) with br_fft_kbw.hpp's one-wave-per-job code; the other
-// waves only stream the key through the LDS ring, so a single gate gets the
-// shared-key pipeline at the latency of one rotating wave. Outputs are
-// bit-identical to k_gate_lvl1_fft (same key switch, same rotation
-// arithmetic).
+// Plain per-gate form with the key bundle at lvl1, one gate per workgroup of
+// eight waves on br_fft_pw.hpp's rotation: four transform waves and four that
+// help with the products and the roots (MUX/NMUX: two jobs of four transform
+// waves). Same key switch and rotation as the batched form, so the outputs are
+// the same words. One NAND of the lvl1 API took 3.80 ms with the rotation on a
+// single wave and the others only streaming the key; now 1.23 ms (MUX 4.40 ->
+// 1.84 ms).
 template <bool MUX>
-__global__ __launch_bounds__(512, 1) void k_gate_lvl1_kbw(
+using GateShape = PwShape<lvl1param, MUX ? 2 : 1, 1, 1, 8, MUX ? 0 : 4>;
+
+// coefficient i of SampleExtractIndex<0> of job `job` (its components lie in
+// the digit 0 buffers after rotate())
+template <class S>
+__device__ __forceinline__ uint32_t gate_sample(const PwWave<S>& w, int job, int i)
+{
+    const uint32_t* a = reinterpret_cast<const uint32_t*>(w.buf(job, 0, 0));
+    if (i == S::N) return reinterpret_cast<const uint32_t*>(w.buf(job, 1, 0))[0];
+    return i == 0 ? a[0] : 0u - a[S::N - i];
+}
+
+// lvl1 API (IKS then BR): MUX/NMUX run c + t - mu and -c + f - mu.
+template <bool MUX>
+__global__ __launch_bounds__(512, 2) void k_gate_lvl1_pw(
     uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
     int32_t cb, uint32_t offset, int32_t mux_sign, const uint32_t* ksk,
     FourierKeys<lvl1param> K)
 {
     using P = lvl1param;
-    constexpr int C = 8, NJ = MUX ? 2 : 1;
-    constexpr int N = P::n, H = N / 2, R = H / 64, n0 = lvl0param::n;
-    constexpr int NT = 64 * C;
+    using S = GateShape<MUX>;
+    static_assert(S::NT == 512, "eight waves");
+    constexpr int N = P::n, n0 = lvl0param::n;
     constexpr uint32_t mu = static_cast<uint32_t>(P::μ);
     constexpr uint32_t rnd = kMaskRound<P>;
-    __shared__ KbwShared<C> sm;
-    __shared__ uint32_t sh_tl0[NJ][kTlwe0Pad];
-    __shared__ uint32_t sh_res[MUX ? 2 : 1][MUX ? N + 1 : 1];
-    const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int t = threadIdx.x;
-    for (int i = t; i < 64; i += NT) {
-        sm.twl[i] = K.fft.twl[i];
-        sm.tws[i] = K.fft.tws[i];
-    }
-    for (int i = t; i < 64; i += NT) {
-        sm.tw64[i] = K.fft.tw64[i];
-        sm.e2n_lo[i] = K.e2n[i];
-    }
-    for (int i = t; i < R; i += NT) sm.cr[i] = K.fft.cr[i];
-    for (int i = t; i < 2 * N / 64; i += NT) sm.e2n_hi[i] = K.e2n[64 * i];
-    // key switch over all eight waves (the transform scratch is free yet and
-    // holds the partial sums)
-    uint32_t* const red = reinterpret_cast<uint32_t*>(&sm.scratch[0][0]);
+    __shared__ PwShared<S> sm;
+    __shared__ uint32_t sh_tl0[S::J][kTlwe0Pad];
+    PwWave<S> w(sm, K, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
+    w.load_tables(threadIdx.x);
+    // key switch over all eight waves (MUX: four per rotation input), partial
+    // sums in the transform buffers
+    uint32_t* const red = reinterpret_cast<uint32_t*>(&sm.buf[0][0]);
     if constexpr (MUX) {
-        // job 0: c + t - mu ; job 1: -c + f - mu (both AND-like, +-mu out)
-        const int job = slot >> 2;
+        const int job = w.wave >> 2;
         key_switch_waves<TFHEpp::lvl10param, false, 4>(
             sh_tl0[job], inc, job == 0 ? in1 : in0, job == 0 ? 1 : -1, 1, 0u - mu, ksk,
-            red + job * 4 * (n0 + 1), slot & 3, t & 63);
+            red + job * 4 * (n0 + 1), w.wave & 3, w.lane);
     }
     else {
         key_switch_waves<TFHEpp::lvl10param, false, 8>(sh_tl0[0], in0, in1, ca, cb, offset, ksk,
-                                                       red, slot, t & 63);
+                                                       red, w.wave, w.lane);
     }
     __syncthreads();
-#pragma unroll
-    for (int job = 0; job < NJ; job++) {
-        for (int i = t; i <= n0; i += NT) {
-            if (i < n0)
-                sm.abar[job][i] = static_cast<uint16_t>(mod_switch<P>(sh_tl0[job][i] + rnd));
-            else
-                sm.bar[job] = 2 * N - mod_switch<P>(sh_tl0[job][n0]);
-        }
-    }
+    const uint32_t* const tl = sh_tl0[w.slot];
+    auto abar = [&](int i) -> uint32_t {
+        return __builtin_amdgcn_readfirstlane(mod_switch<P>(tl[i] + rnd));
+    };
+    w.rotate(true, __builtin_amdgcn_readfirstlane(2 * N - mod_switch<P>(tl[n0])), mu, abar);
     __syncthreads();
-    if (slot < NJ) {
-        uint32_t acc[2][16];
-        blind_rotate_kbw<C>(sm, slot, mu, acc, K.bk);
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            AccStore<P> a;
-#pragma unroll
-            for (int r = 0; r < 16; r++) a.reg[r] = acc[j][r];
-            sample_extract_store<P>(a, j, MUX ? sh_res[slot] : out);
+    for (int i = threadIdx.x; i <= N; i += S::NT) {
+        uint32_t v = gate_sample(w, 0, i);
+        if constexpr (MUX) {
+            v += gate_sample(w, 1, i) + (i == N ? mu : 0u);
+            if (mux_sign < 0) v = 0u - v;
         }
-    }
-    else {
-        KbwKeyPipe<C> pipe(sm, slot, t & 63, K.bk);
-        pipe.run_loader_only();
-    }
-    if constexpr (MUX) {
-        __syncthreads();
-        for (int i = t; i <= N; i += NT) {
-            uint32_t v = sh_res[0][i] + sh_res[1][i];
-            if (i == N) v += mu;
-            out[i] = mux_sign > 0 ? v : 0u - v;
-        }
+        out[i] = v;
     }
 }
 
-// Plain per-gate form with the key bundle, lvl0 API (BR then IKS), on the
-// same eight-wave organisation as k_gate_lvl1_kbw: waves 0 (and 1) rotate,
-// the others stream the key; then all eight waves key-switch. Outputs are
-// bit-identical to k_gate_lvl01_fft.
+// lvl0 API (BR then IKS): the pre-added lvl0 inputs are mod-switched as they
+// are read; the extracted samples wait in LDS for the key switch.
 template <bool MUX, bool SUBSET>
-__global__ __launch_bounds__(512, 1) void k_gate_lvl01_kbw(
+__global__ __launch_bounds__(512, 2) void k_gate_lvl01_pw(
     uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
     int32_t cb, uint32_t offset, int32_t mux_sign, uint32_t tv_mu, const uint32_t* ksk,
     FourierKeys<lvl1param> K)
 {
     using P = lvl1param;
-    constexpr int C = 8, NJ = MUX ? 2 : 1;
-    constexpr int N = P::n, H = N / 2, R = H / 64, n0 = lvl0param::n;
-    constexpr int NT = 64 * C;
+    using S = GateShape<MUX>;
+    constexpr int N = P::n, n0 = lvl0param::n;
     constexpr uint32_t mu = static_cast<uint32_t>(P::μ);
     constexpr uint32_t mu0 = static_cast<uint32_t>(lvl0param::μ);
     constexpr uint32_t rnd = kMaskRound<P>;
-    __shared__ KbwShared<C> sm;
-    __shared__ uint32_t sh_res[NJ][N + 4];
-    const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int t = threadIdx.x;
-    for (int i = t; i < 64; i += NT) {
-        sm.twl[i] = K.fft.twl[i];
-        sm.tws[i] = K.fft.tws[i];
-    }
-    for (int i = t; i < 64; i += NT) {
-        sm.tw64[i] = K.fft.tw64[i];
-        sm.e2n_lo[i] = K.e2n[i];
-    }
-    for (int i = t; i < R; i += NT) sm.cr[i] = K.fft.cr[i];
-    for (int i = t; i < 2 * N / 64; i += NT) sm.e2n_hi[i] = K.e2n[64 * i];
-    // the pre-added lvl0 inputs (as k_gate_lvl01_fft), mod-switched
-#pragma unroll
-    for (int job = 0; job < NJ; job++) {
-        const uint32_t* a = MUX ? inc : in0;
-        const uint32_t* b = MUX ? (job == 0 ? in1 : in0) : in1;
-        const int32_t sa = MUX ? (job == 0 ? 1 : -1) : ca;
-        const int32_t sb = MUX ? 1 : cb;
-        const uint32_t off = MUX ? 0u - mu0 : offset;
-        for (int i = t; i <= n0; i += NT) {
-            uint32_t v = static_cast<uint32_t>(sa) * a[i] + static_cast<uint32_t>(sb) * b[i];
-            if (i < n0)
-                sm.abar[job][i] = static_cast<uint16_t>(mod_switch<P>(v + rnd));
-            else
-                sm.bar[job] = 2 * N - mod_switch<P>(v + off);
-        }
-    }
+    __shared__ PwShared<S> sm;
+    __shared__ uint32_t sh_res[S::J][N + 4];
+    PwWave<S> w(sm, K, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
+    w.load_tables(threadIdx.x);
     __syncthreads();
-    if (slot < NJ) {
-        uint32_t acc[2][16];
-        blind_rotate_kbw<C>(sm, slot, tv_mu, acc, K.bk);
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            AccStore<P> r;
-#pragma unroll
-            for (int k = 0; k < 16; k++) r.reg[k] = acc[j][k];
-            sample_extract_store<P>(r, j, sh_res[slot]);
-        }
-    }
-    else {
-        KbwKeyPipe<C> pipe(sm, slot, t & 63, K.bk);
-        pipe.run_loader_only();
-    }
+    const uint32_t* a = MUX ? inc : in0;
+    const uint32_t* b = MUX ? (w.slot == 0 ? in1 : in0) : in1;
+    const uint32_t sa = static_cast<uint32_t>(MUX ? (w.slot == 0 ? 1 : -1) : ca);
+    const uint32_t sb = static_cast<uint32_t>(MUX ? 1 : cb);
+    const uint32_t off = MUX ? 0u - mu0 : offset;
+    auto abar = [&](int i) -> uint32_t {
+        return __builtin_amdgcn_readfirstlane(mod_switch<P>(sa * a[i] + sb * b[i] + rnd));
+    };
+    w.rotate(true, __builtin_amdgcn_readfirstlane(2 * N - mod_switch<P>(sa * a[n0] + sb * b[n0] + off)),
+             tv_mu, abar);
     __syncthreads();
-    // key switch over all eight waves, partial sums in the transform scratch
-    uint32_t* const red = reinterpret_cast<uint32_t*>(&sm.scratch[0][0]);
+#pragma unroll
+    for (int job = 0; job < S::J; job++)
+        for (int i = threadIdx.x; i <= N; i += S::NT) sh_res[job][i] = gate_sample(w, job, i);
+    __syncthreads();
+    uint32_t* const red = reinterpret_cast<uint32_t*>(&sm.buf[0][0]);
     if constexpr (MUX)
         key_switch_waves<TFHEpp::lvl10param, SUBSET, 8>(out, sh_res[0], sh_res[1], mux_sign,
                                                         mux_sign, mux_sign > 0 ? mu : 0u - mu, ksk,
-                                                        red, slot, t & 63);
+                                                        red, w.wave, w.lane);
     else
         key_switch_waves<TFHEpp::lvl10param, SUBSET, 8>(out, sh_res[0], nullptr, 1, 0, 0u, ksk,
-                                                        red, slot, t & 63);
+                                                        red, w.wave, w.lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -801,12 +752,11 @@ void launch_gate_lvl1_fft(bool kb, bool mux, uint32_t* out, const uint32_t* in0,
     hipLaunchKernelGGL((k_gate_lvl1_fft<KBV, MUXV>), grid, block, 0, st, out, in0, in1, inc, \
                        ca, cb, offset, mux_sign, ksk, K)
     if (kb) {
-        // key bundle: the one-wave rotation with seven key-loading waves
         if (mux)
-            hipLaunchKernelGGL((k_gate_lvl1_kbw<true>), grid, dim3(512), 0, st, out, in0, in1, inc,
+            hipLaunchKernelGGL((k_gate_lvl1_pw<true>), grid, dim3(512), 0, st, out, in0, in1, inc,
                                ca, cb, offset, mux_sign, ksk, K);
         else
-            hipLaunchKernelGGL((k_gate_lvl1_kbw<false>), grid, dim3(512), 0, st, out, in0, in1,
+            hipLaunchKernelGGL((k_gate_lvl1_pw<false>), grid, dim3(512), 0, st, out, in0, in1,
                                inc, ca, cb, offset, mux_sign, ksk, K);
     }
     else {
@@ -824,9 +774,8 @@ void launch_gate_lvl01_fft(bool kb, bool mux, bool subset, uint32_t* out, const 
     hipLaunchKernelGGL((k_gate_lvl01_fft<KBV, MUXV, SUB>), dim3(1), dim3(512), 0, \
                        st, out, in0, in1, inc, ca, cb, offset, mux_sign, tv_mu, ksk, K)
     if (kb) {
-        // key bundle: the one-wave rotation with seven key-streaming waves
 #define CUFHE_K01(MUXV, SUB)                                                                     \
-    hipLaunchKernelGGL((k_gate_lvl01_kbw<MUXV, SUB>), dim3(1), dim3(512), 0, st, out, in0, in1, \
+    hipLaunchKernelGGL((k_gate_lvl01_pw<MUXV, SUB>), dim3(1), dim3(512), 0, st, out, in0, in1, \
                        inc, ca, cb, offset, mux_sign, tv_mu, ksk, K)
         if (mux) {
             if (subset) CUFHE_K01(true, true); else CUFHE_K01(true, false);
