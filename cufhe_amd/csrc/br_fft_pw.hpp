@@ -1,10 +1,10 @@
-// Key-bundle blind rotation with the digit transforms of a job spread over
-// several waves and the multiply-accumulate split over all waves by spectrum
-// bins.
+// Blind rotation with the digit transforms of a job spread over several waves
+// and the multiply-accumulate split over all waves by spectrum bins: the key
+// bundle at lvl1 and lvl2, CMUX keys (one TRGSW per key bit) at lvl1.
 //
-// Arithmetic: br_fft.hpp's key-bundle step (reference
-// include/gatebootstrapping_gpu.cuh:895-1033 AccumulateKeyBundle and
-// :1335-1429 the drivers). At lvl2 operation for operation, so the outputs are
+// Arithmetic: br_fft.hpp's steps (reference
+// include/gatebootstrapping_gpu.cuh:895-1033 AccumulateKeyBundle, :69-221
+// Accumulate, and :1335-1429 the drivers). At lvl2 operation for operation, so the outputs are
 // bit-identical to k_br_fft. At lvl1 the external product is an integer that
 // FP64 leaves within a small fraction of a unit, so any order of operations
 // rounds to the same words: there the transforms are fft512.hpp's and
@@ -22,6 +22,8 @@
 //  3. inverse: wave qi = 0 of (job, j) transforms component j's output back,
 //     rounds, and hands the next digits to its partner waves through their idle
 //     buffers; a partner (or the wave itself) prepares the next step's roots.
+//     With CMUX keys it adds to the accumulator it keeps and publishes that in
+//     LDS, where phase 1 reads it rotated.
 // What bounds it: FP64 issue and LDS traffic, about equally, over the whole
 // CU. (An LDS KiB costs a CU 5.7 ns written and 3.2 ns read, a wave's FP64
 // instruction 0.5 ns; FP64 MFMA runs on the same pipe as the vector FMAs.)
@@ -36,7 +38,7 @@ namespace cufhe_amd {
 // digits go through phases 1-2 in PASSES passes (fewer digit buffers in LDS,
 // the sums stay in VGPRs between them); PF key blocks (three values) are in
 // flight per lane.
-template <class P_, int J_, int PASSES_, int DPW_, int PF_, int HELP_ = 0>
+template <class P_, int J_, int PASSES_, int DPW_, int PF_, int HELP_ = 0, bool KB_ = true>
 struct PwShape {
     using P = P_;
     using T = typename P::T;
@@ -53,19 +55,24 @@ struct PwShape {
     static constexpr int BPL = W > R ? 1 : R / W;   // registers (64-bin groups) per wave
     static constexpr int BLK = QD * 4;              // key blocks per pass and register
     static constexpr int NB = BPL * BLK;            // key blocks per pass
-    static constexpr int STEPS = lvl0param::n / 2;
+    static constexpr bool KB = KB_;
+    static constexpr int NM = KB ? 3 : 1;  // key values of a block: the bundle's members
+    static constexpr int STEPS = KB ? lvl0param::n / 2 : lvl0param::n;
     // root sets in LDS: lvl1 forms X^(a0+a1) as a product, lvl2 reads it from the table
     static constexpr int NX = kLvl1 ? 2 : 3;
-    // digit words per lane: lvl1 packs both digits of two coefficients
-    static constexpr int WORDS = kLvl1 ? R : R * PASSES;
+    // digit words per lane: lvl1 one for both digits of two coefficients, lvl2
+    // one for three digits of a coefficient
+    static constexpr int WORDS = kLvl1 ? R : 2 * R;
     static constexpr bool kPrio = J > 1;  // several waves per SIMD meet at the barriers
     // all key blocks of a step in flight before phase 2 (else PF ahead, rolling)
     static constexpr bool kFull = PASSES == 1 && PF == NB;
     // the roots of a job in the idle ends of its digit 1 buffers instead of an array
-    static constexpr bool kTail = kLvl1 && QW == 2 && HELP == 0;
+    static constexpr bool kTail = KB && kLvl1 && QW == 2 && HELP == 0;
+    static constexpr bool kBase = KB && !kTail;
     static constexpr int TAB = kLvl1 ? fft512::kTabWords : 3 * 64;
     static_assert(QW * DPW == QD && QD * PASSES == L && JL * SETS == J, "shape");
-    static_assert(kLvl1 || DPW == 1, "lvl2 packs one digit per word half");
+    static_assert(kLvl1 || (DPW == 1 && L == 4 && P::Bgbit == 10), "lvl2 digit words");
+    static_assert(KB || (kLvl1 && PASSES == 1), "CMUX keys: lvl1");
     static_assert(HELP == 0 || HELP >= 2 * J, "two root waves per job");
     static_assert(!kFull || kLvl1, "the next step's keys are loaded in fft512's hooks");
     static_assert((W > R ? W % R == 0 : R % W == 0) && NB % PF == 0, "even split");
@@ -77,6 +84,34 @@ struct PwShared {
     cplx base[S::kTail ? 1 : S::J][S::NX][S::G][S::kTail ? 1 : 64];                          // E[a (1 - 4 kb)] of a0, a1 (, a0 + a1)
     cplx tab[S::TAB];                                          // transform tables
     uint32_t a[S::J][S::NX];
+    typename S::T acc[S::KB ? 1 : S::J][2][S::KB ? 1 : S::N];  // CMUX keys: the accumulators
+};
+
+// The lvl0 mask of a job: load(i) starts a coefficient on its way, value()
+// mod-switches it to [0, 2N) (wave-uniform) a step later, so no wave waits for
+// the load. ca * in0 + cb * in1 in global memory (in1 may be null), or words
+// in LDS.
+struct PwMask {
+    const uint32_t* in0;
+    const uint32_t* in1;
+    uint32_t ca, cb;
+    struct Raw {
+        uint32_t x, y;
+    };
+    __device__ __forceinline__ Raw load(int i) const { return Raw{in0[i], in1 ? in1[i] : 0u}; }
+    __device__ __forceinline__ uint32_t sum(Raw r) const { return ca * r.x + cb * r.y; }
+    template <class P>
+    __device__ __forceinline__ uint32_t value(Raw r) const
+    {
+        return __builtin_amdgcn_readfirstlane(mod_switch<P>(sum(r) + kMaskRound<P>));
+    }
+    // the rotation by the body (offset added)
+    template <class P>
+    __device__ __forceinline__ uint32_t body(uint32_t offset) const
+    {
+        return __builtin_amdgcn_readfirstlane(2 * P::n -
+                                              mod_switch<P>(sum(load(lvl0param::n)) + offset));
+    }
 };
 
 template <class S>
@@ -84,6 +119,7 @@ struct PwWave {
     using P = typename S::P;
     using T = typename S::T;
     static constexpr int N = S::N, H = S::H, R = S::R, L = S::L;
+    static constexpr int kPer = S::WORDS / R;  // words of a coefficient pair
     PwShared<S>& sm;
     const FourierKeys<P>& K;
     const int wave, lane;
@@ -138,36 +174,42 @@ struct PwWave {
         }
     }
 
-    // The words of digit wave q_ for coefficients lo (r) and hi (R + r).
-    __device__ __forceinline__ static uint32_t pack(T lo, T hi, int q_, int pass)
+    // Digit words of coefficients lo (r) and hi (R + r) for the wave qi = 0
+    // (own) and for its partners. The digits are fields of c + offset less half
+    // their range; with each field's top bit flipped they read as signed.
+    // lvl1: both digits are the bytes 3 and 2, one word for two coefficients.
+    // lvl2: four fields of 10 bits; the high word holds digits 0-2, bits 24-55
+    // hold digits 1-3.
+    struct Words {
+        uint32_t own[2], partner[2];
+    };
+    __device__ __forceinline__ static Words pack(T lo, T hi)
     {
         if constexpr (S::kLvl1) {
-            // bytes 3 and 2 of c + offset are the digits + 128
             const uint32_t a = lo + Gadget<P>::kOffset, b = hi + Gadget<P>::kOffset;
-            return ((a >> 16) | (b & 0xffff0000u)) ^ 0x80808080u;
+            const uint32_t w = ((a >> 16) | (b & 0xffff0000u)) ^ 0x80808080u;
+            return Words{{w, 0u}, {w, 0u}};
         }
         else {
-            const int q = pass * S::QD + q_;
-            return (static_cast<uint32_t>(Gadget<P>::digit(lo, q)) & 0xffffu) |
-                   (static_cast<uint32_t>(Gadget<P>::digit(hi, q)) << 16);
+            constexpr uint64_t flip = (1ull << 63) | (1ull << 53) | (1ull << 43) | (1ull << 33);
+            const uint64_t a = (lo + Gadget<P>::kOffset) ^ flip, b = (hi + Gadget<P>::kOffset) ^ flip;
+            return Words{{static_cast<uint32_t>(a >> 32), static_cast<uint32_t>(b >> 32)},
+                         {static_cast<uint32_t>(a >> 24), static_cast<uint32_t>(b >> 24)}};
         }
     }
-    // folded digit m of this wave (lvl1: gadget digit qi * DPW + m) at register r
+    // folded digit m of this wave (gadget digit (pass QW + qi) DPW + m) at register r
     __device__ __forceinline__ cplx digits(int r, int pass, int m) const
     {
+        const int q = (pass * S::QW + qi) * S::DPW + m;
+        auto field = [](uint32_t w, int at, int bits) {
+            return static_cast<double>(static_cast<int32_t>(__builtin_amdgcn_sbfe(w, at, bits)));
+        };
         if constexpr (S::kLvl1) {
-            const uint32_t sh = 8 * (1 - (qi * S::DPW + m));
-            return cplx{static_cast<double>(static_cast<int32_t>(__builtin_amdgcn_sbfe(words[r], sh, 8))),
-                        static_cast<double>(
-                            static_cast<int32_t>(__builtin_amdgcn_sbfe(words[r], sh + 16, 8)))};
+            return cplx{field(words[r], 8 * (1 - q), 8), field(words[r], 24 - 8 * q, 8)};
         }
         else {
-            uint32_t u = words[r];
-#pragma unroll
-            for (int p = 1; p < S::PASSES; p++)
-                if (p == pass) u = words[p * R + r];
-            const int32_t w = static_cast<int32_t>(u);
-            return cplx{static_cast<double>(static_cast<int16_t>(w)), static_cast<double>(w >> 16)};
+            const int at = qi == 0 ? 22 - 10 * q : 30 - 10 * q;
+            return cplx{field(words[2 * r], at, 10), field(words[2 * r + 1], at, 10)};
         }
     }
     __device__ __forceinline__ void init_digits(uint32_t bar, T mu)
@@ -177,8 +219,9 @@ struct PwWave {
             const int i0 = lane + 64 * r;
             const T lo = j == 0 ? T(0) : test_vector_coef<P>(i0, bar, mu);
             const T hi = j == 0 ? T(0) : test_vector_coef<P>(i0 + H, bar, mu);
+            const Words v = pack(lo, hi);
 #pragma unroll
-            for (int p = 0; p < S::WORDS / R; p++) words[p * R + r] = pack(lo, hi, qi, p);
+            for (int k = 0; k < kPer; k++) words[kPer * r + k] = qi == 0 ? v.own[k] : v.partner[k];
         }
     }
 
@@ -234,7 +277,7 @@ struct PwWave {
     // Key block b of a pass: register dd, digit, component, output column; its
     // three bundle members.
     struct KeyBlk {
-        cplx k[3];
+        cplx k[S::NM];
     };
     __device__ __forceinline__ KeyBlk load_key(int step, int pass, int b, int d0) const
     {
@@ -244,7 +287,7 @@ struct PwWave {
         const uint32_t st = __builtin_amdgcn_readfirstlane(step);
         const uint32_t in_step = __builtin_amdgcn_readfirstlane(
             ((comp * L + pass * S::QD + ql) * 2 + col) * H + (d0 + dd) * 64);
-        const uint64_t u = reinterpret_cast<uint64_t>(K.bk + st * (3 * TS) + in_step);
+        const uint64_t u = reinterpret_cast<uint64_t>(K.bk + st * (S::NM * TS) + in_step);
         using gbytes = const __attribute__((address_space(1))) char*;
         const gbytes p = (gbytes)(
             (static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(u >> 32))) << 32) |
@@ -255,15 +298,16 @@ struct PwWave {
             const v2 v = *(const __attribute__((address_space(1))) v2*)(p + e * TS * sizeof(cplx) + off);
             return cplx{v.x, v.y};
         };
-        return KeyBlk{{at(0), at(1), at(2)}};
+        KeyBlk v;
+#pragma unroll
+        for (int e = 0; e < S::NM; e++) v.k[e] = at(e);
+        return v;
     }
 
-    // The rotation of the workgroup's jobs. abar(i): this wave's job's
-    // mod-switched mask coefficient i (wave-uniform). live: whether this
-    // wave's job exists. At the end the buffer of (job, j, digit 0) holds the N
+    // The rotation of the workgroup's jobs. mask: that of this wave's job, bar:
+    // its body's rotation. live: whether this wave's job exists. At the end the buffer of (job, j, digit 0) holds the N
     // coefficients of component j (visible to the wave with qi = 0).
-    template <class Abar>
-    __device__ __forceinline__ void rotate(bool live, uint32_t bar, T mu, Abar&& abar)
+    __device__ __forceinline__ void rotate(bool live, uint32_t bar, T mu, const PwMask& mask)
     {
         constexpr int PF = S::PF, NB = S::NB;
         const int set = S::W > R ? wave / R : 0;
@@ -271,19 +315,35 @@ struct PwWave {
         const bool fft = live && qi >= 0;
         cplx* const mine = buf(slot, j, (qi < 0 ? 0 : qi) * S::DPW);
         const fft512::Slots slots = fft512::Slots::of(lane);
-        uint32_t na0 = 0, na1 = 0;
-        if (fft) init_digits(bar, mu);
-        Gathered roots;
-        if (live && rooter) {
-            roots = gather(abar(0), abar(1));
-            put(roots);
-            na0 = abar(2);
-            na1 = abar(3);
+        PwMask::Raw na0{0, 0}, na1{0, 0};  // the next step's mask coefficients
+        T acc[S::KB ? 1 : 2 * R];  // CMUX keys: this wave's component
+        if constexpr (S::KB) {
+            if (fft) init_digits(bar, mu);
+        }
+        else {
+            if (fft && qi == 0) {
+#pragma unroll
+                for (int r = 0; r < 2 * R; r++) {
+                    const int i = AccStore<P>::coef_index(r, lane);
+                    acc[r] = j == 0 ? T(0) : test_vector_coef<P>(i, bar, mu);
+                    sm.acc[slot][j][i] = acc[r];
+                }
+            }
+            if (fft) na0 = mask.load(0);
+        }
+        cplx tail_root;  // kTail: the next root until its place is free
+        if (S::KB && live && rooter) {
+            const Gathered first =
+                gather(mask.value<P>(mask.load(0)), mask.value<P>(mask.load(1)));
+            put(first);
+            tail_root = first.v[0][0];
+            na0 = mask.load(2);
+            na1 = mask.load(3);
         }
         auto next_mask = [&](int it) {
             if (it + 2 < S::STEPS) {
-                na0 = abar(2 * it + 4);
-                na1 = abar(2 * it + 5);
+                na0 = mask.load(2 * it + 4);
+                na1 = mask.load(2 * it + 5);
             }
         };
         KeyBlk kv[PF];
@@ -299,23 +359,28 @@ struct PwWave {
         for (int it = 0; it < S::STEPS; it++) {
             // the last blocks of a step prefetch the next step's first ones
             const int next = it + 1 < S::STEPS ? it + 1 : it;
-            // W_8^(a d) of this step (scalar loads, long before their use)
+            // W_8^(a d) of this step: scalar loads, at lvl1 long before their use
+            // (at lvl2 the transforms need the SGPRs)
             cplx w8[S::BPL][S::JL][S::NX];
+            auto load_w8 = [&]() {
 #pragma unroll
-            for (int jl = 0; jl < S::JL; jl++)
+                for (int jl = 0; jl < S::JL; jl++)
 #pragma unroll
-                for (int m = 0; m < S::NX; m++) {
-                    const uint32_t a = __builtin_amdgcn_readfirstlane(sm.a[set * S::JL + jl][m]);
+                    for (int m = 0; m < S::NX; m++) {
+                        const uint32_t a = __builtin_amdgcn_readfirstlane(sm.a[set * S::JL + jl][m]);
 #pragma unroll
-                    for (int dd = 0; dd < S::BPL; dd++) {
-                        const int e = (a * static_cast<uint32_t>(d0 + dd)) & 7u;
-                        w8[dd][jl][m] = cplx{kW8[e][0], kW8[e][1]};
+                        for (int dd = 0; dd < S::BPL; dd++) {
+                            const int e = (a * static_cast<uint32_t>(d0 + dd)) & 7u;
+                            w8[dd][jl][m] = cplx{kW8[e][0], kW8[e][1]};
+                        }
                     }
-                }
+            };
+            if constexpr (S::KB && S::kLvl1) load_w8();
             const bool more = it + 1 < S::STEPS;
-            if (S::HELP && live && rooter && more) {
+            Gathered roots;
+            if (S::KB && S::HELP && live && rooter && more) {
                 // helpers gather the next step's roots while the others transform
-                roots = gather(na0, na1);
+                roots = gather(mask.value<P>(na0), mask.value<P>(na1));
                 next_mask(it);
             }
             cplx s[S::BPL][S::JL][2];
@@ -328,6 +393,28 @@ struct PwWave {
                 const bool last = pass + 1 == S::PASSES;
                 const int after = last ? next : it;
                 const int after_pass = last ? 0 : pass + 1;
+                if constexpr (!S::KB) {
+                    // digits of (X^a - 1) acc
+                    if (fft) {
+                        const uint32_t a = mask.value<P>(na0);
+                        if (more) na0 = mask.load(it + 1);
+                        const T* const src = sm.acc[slot][j];
+#pragma unroll
+                        for (int r = 0; r < R; r++) {
+                            const int i = lane + 64 * r;
+                            // X^a acc at i: acc[(i - a) mod N], negated where bit
+                            // log N of i - a (mod 2N) is set
+                            auto rotated = [&](int k) {
+                                const uint32_t u = static_cast<uint32_t>(k) - a;
+                                const uint32_t neg = 0u - ((u >> P::nbit) & 1u);
+                                return (static_cast<uint32_t>(src[u & (N - 1)]) ^ neg) - neg;
+                            };
+                            const Words v = pack(static_cast<T>(rotated(i)) - src[i],
+                                                 static_cast<T>(rotated(i + H)) - src[i + H]);
+                            words[r] = v.own[0];
+                        }
+                    }
+                }
                 if (fft) {
                     if constexpr (S::kLvl1) {
                         cplx z[S::DPW][8];
@@ -376,7 +463,7 @@ struct PwWave {
                     }
                 }
                 if constexpr (S::kTail)
-                    if (live && rooter) lds_store(&mine[H + lane], roots.v[0][0]);
+                    if (live && rooter) lds_store(&mine[H + lane], tail_root);
                 if (!fft && S::kFull && !early) {
                     // no job: the wave still multiplies for the others
 #pragma unroll
@@ -385,6 +472,7 @@ struct PwWave {
                 // X^a - 1 at this wave's bins; the roots were published a barrier ago
                 cplx x[S::BPL][S::JL][3];
                 auto make_x = [&]() {
+                    if constexpr (!S::kLvl1) load_w8();
 #pragma unroll
                 for (int dd = 0; dd < S::BPL; dd++)
 #pragma unroll
@@ -399,7 +487,7 @@ struct PwWave {
                         for (int m = 0; m < 3; m++) xx[m].x -= 1.0;
                     }
                 };
-                if constexpr (!S::kTail) make_x();
+                if constexpr (S::kBase) make_x();
                 __syncthreads();  // digit spectra are in LDS
                 if constexpr (S::kTail) make_x();
                 // the spectra of a (digit, component) are loaded while the one
@@ -435,10 +523,13 @@ struct PwWave {
                                                              : load_key(after, after_pass, i + PF - NB, d0);
 #pragma unroll
                                 for (int jl = 0; jl < S::JL; jl++) {
-                                    cplx k = {comp == col ? hq : 0.0, 0.0};
-                                    cmac(k, cur.k[2], x[dd][jl][1]);
-                                    cmac(k, cur.k[1], x[dd][jl][0]);
-                                    cmac(k, cur.k[0], x[dd][jl][2]);
+                                    cplx k = cur.k[0];
+                                    if constexpr (S::KB) {
+                                        k = cplx{comp == col ? hq : 0.0, 0.0};
+                                        cmac(k, cur.k[2], x[dd][jl][1]);
+                                        cmac(k, cur.k[1], x[dd][jl][0]);
+                                        cmac(k, cur.k[0], x[dd][jl][2]);
+                                    }
                                     cmac(s[dd][jl][col], D[n & 1][jl], k);
                                 }
                                 // the loads of later blocks stay behind this block's products
@@ -457,9 +548,13 @@ struct PwWave {
                     for (int col = 0; col < 2; col++)
                         lds_store(&buf(set * S::JL + jl, col, 0)[(d0 + dd) * 64 + lane], s[dd][jl][col]);
             __syncthreads();  // output spectra are in the digit 0 buffers
-            if (S::HELP == 0 && live && rooter && more) {
-                roots = gather(na0, na1);
-                next_mask(it);
+            if (S::KB && S::HELP == 0 && live && rooter && more) {
+                if constexpr (!S::kLvl1) {  // an idle partner wave, short of VGPRs
+                    na0 = mask.load(2 * it + 2);
+                    na1 = mask.load(2 * it + 3);
+                }
+                roots = gather(mask.value<P>(na0), mask.value<P>(na1));
+                if constexpr (S::kLvl1) next_mask(it);
             }
             // (behind the roots' loads: they return in order)
             if (S::kFull && early) {
@@ -498,17 +593,29 @@ struct PwWave {
                     else
                         return double_to_torus<T>(v * (kTorusScale<T> / H));
                 };
-                if (more) {
+                if constexpr (!S::KB) {
+                    T* const res = more ? sm.acc[slot][j] : reinterpret_cast<T*>(mine);
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        acc[r] += torus(z[r].x, r);
+                        acc[R + r] += torus(z[r].y, r);
+                        res[lane + 64 * r] = acc[r];
+                        res[lane + 64 * r + H] = acc[R + r];
+                    }
+                    wave_lds_sync();
+                }
+                else if (more) {
 #pragma unroll
                     for (int r = 0; r < R; r++) {
                         const T lo = torus(z[r].x, r), hi = torus(z[r].y, r);
+                        const Words v = pack(lo, hi);
 #pragma unroll
-                        for (int p = 0; p < S::WORDS / R; p++) {
-                            words[p * R + r] = pack(lo, hi, 0, p);
+                        for (int k = 0; k < kPer; k++) {
+                            words[kPer * r + k] = v.own[k];
 #pragma unroll
                             for (int q = 1; q < S::QW; q++)
-                                reinterpret_cast<uint32_t*>(buf(slot, j, q * S::DPW))[(p * R + r) * 64 + lane] =
-                                    pack(lo, hi, q, p);
+                                reinterpret_cast<uint32_t*>(buf(slot, j, q * S::DPW))[(kPer * r + k) * 64 + lane] =
+                                    v.partner[k];
                         }
                     }
                 }
@@ -522,10 +629,13 @@ struct PwWave {
                     wave_lds_sync();
                 }
             }
-            if (live && rooter && more) put(roots);
+            if (S::KB && live && rooter && more) {
+                put(roots);
+                if constexpr (S::kTail) tail_root = roots.v[0][0];
+            }
             if (more) {
                 __syncthreads();  // next digits and roots are ready
-                if (live && qi > 0) {
+                if (S::KB && live && qi > 0) {
 #pragma unroll
                     for (int w = 0; w < S::WORDS; w++)
                         words[w] = reinterpret_cast<const uint32_t*>(mine)[w * 64 + lane];

@@ -167,8 +167,6 @@ __global__ __launch_bounds__(S::NT, WPE) void k_br_fft_pw(const BrJob* __restric
 {
     using P = typename S::P;
     using T = typename S::T;
-    constexpr int n0 = lvl0param::n;
-    constexpr uint32_t rnd = kMaskRound<P>;
     __shared__ PwShared<S> sm;
     PwWave<S> w(sm, K, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
     w.load_tables(threadIdx.x);
@@ -178,82 +176,20 @@ __global__ __launch_bounds__(S::NT, WPE) void k_br_fft_pw(const BrJob* __restric
         const int raw = grp * S::J + w.slot;
         const bool live = raw < njobs;
         const BrJob jb = jobs[live ? raw : njobs - 1];
-        auto pre = [&](int i) -> uint32_t {
-            uint32_t v = static_cast<uint32_t>(jb.ca) * jb.in0[i];
-            if (jb.in1) v += static_cast<uint32_t>(jb.cb) * jb.in1[i];
-            return v;
-        };
-        auto abar = [&](int i) -> uint32_t {
-            return __builtin_amdgcn_readfirstlane(mod_switch<P>(pre(i) + rnd));
-        };
-        const uint32_t bar =
-            __builtin_amdgcn_readfirstlane(2 * S::N - mod_switch<P>(pre(n0) + jb.offset));
-        w.rotate(live, bar, mu, abar);
+        const PwMask mask{jb.in0, jb.in1, static_cast<uint32_t>(jb.ca), static_cast<uint32_t>(jb.cb)};
+        w.rotate(live, mask.body<P>(jb.offset), mu, mask);
         if (live && w.qi == 0)
             pw_store<P>(reinterpret_cast<const T*>(w.buf(w.slot, w.j, 0)), w.j, w.lane,
                         jb.flags & kBrOutTrlwe, static_cast<T*>(jb.out));
     }
 }
 
-// ---------------------------------------------------------------------------
-// Plain per-gate form, lvl0 API (BR-IKS at lvl1; reference
-// src/cufhe_gates_gpu.cu:198-511, src/bootstrap_gpu.cu:1557-1672): lvl0
-// inputs pre-added into the rotation, SampleExtract, key switch lvl1 -> lvl0.
-// MUX/NMUX rotate c + t - mu and -c + f - mu on two wave pairs and key-switch
-// +-(r1 + r0 + mu) in one pass.
-template <bool KB, bool MUX, bool SUBSET>
-__global__ __launch_bounds__(512, 1) void k_gate_lvl01_fft(
-    uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
-    int32_t cb, uint32_t offset, int32_t mux_sign, uint32_t tv_mu, const uint32_t* ksk,
-    FourierKeys<lvl1param> K)
-{
-    using P = lvl1param;
-    constexpr int C = MUX ? 2 : 1;
-    constexpr int N = P::n, H = N / 2, n0 = lvl0param::n;
-    constexpr uint32_t mu = static_cast<uint32_t>(P::μ);
-    constexpr uint32_t mu0 = static_cast<uint32_t>(lvl0param::μ);
-    constexpr int NB = BrShape<P>::NB;
-    __shared__ cplx sh_spec[2 * C][NB * H];
-    __shared__ uint32_t sh_tl0[C][kTlwe0Pad];
-    __shared__ uint32_t sh_res[C][N + 4];
-    __shared__ uint32_t sh_red[8 * (n0 + 1)];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int slot = wave >> 1, j = wave & 1;
-    const int t = threadIdx.x & 127;
-    // waves 0 .. 2C-1 rotate; the others keep step through the rotation's
-    // barriers and then join the key switch (eight waves)
-    const bool rotating = wave < 2 * C;
-    if (rotating) {
-        const uint32_t* a = MUX ? inc : in0;
-        const uint32_t* b = MUX ? (slot == 0 ? in1 : in0) : in1;
-        const int32_t sa = MUX ? (slot == 0 ? 1 : -1) : ca;
-        const int32_t sb = MUX ? 1 : cb;
-        const uint32_t off = MUX ? 0u - mu0 : offset;
-        for (int i = t; i <= n0; i += 128) {
-            uint32_t v = static_cast<uint32_t>(sa) * a[i] + static_cast<uint32_t>(sb) * b[i];
-            if (i == n0) v += off;
-            sh_tl0[slot][i] = v;
-        }
-    }
-    __syncthreads();
-    if (rotating) {
-        AccStore<P> acc;
-        blind_rotate_fft<P, KB>(sh_tl0[slot], tv_mu, acc, j, sh_spec[wave], sh_spec[wave ^ 1], K);
-        sample_extract_store<P>(acc, j, sh_res[slot]);
-    }
-    else {
-        blind_rotate_ghost<P, KB>(K);
-    }
-    __syncthreads();
-    if constexpr (MUX)
-        key_switch_waves<TFHEpp::lvl10param, SUBSET, 8>(out, sh_res[0], sh_res[1], mux_sign,
-                                                        mux_sign, mux_sign > 0 ? mu : 0u - mu, ksk,
-                                                        sh_red, wave, threadIdx.x & 63);
-    else
-        key_switch_waves<TFHEpp::lvl10param, SUBSET, 8>(out, sh_res[0], nullptr, 1, 0, 0u, ksk,
-                                                        sh_red, wave, threadIdx.x & 63);
-}
+// The lvl2 shape: eight waves, one digit polynomial each, two 64-bin groups of
+// the products. Four key blocks (12 KiB) in flight a wave: the phase streams
+// 786 KB of key through the CU's L2 path; eight spill.
+using Lvl2Shape = PwShape<lvl2param, 1, 1, 1, 4>;
 
+// ---------------------------------------------------------------------------
 // SampleExtract + key switch lvl1 -> lvl0 of n TRLWEs (reference SEIandKS,
 // src/keyswitch_gpu.cu:61-68, include/keyswitch_gpu.cuh:52-123), one job per
 // workgroup.
@@ -279,68 +215,16 @@ __global__ __launch_bounds__(512) void k_se_ks_lvl10(uint32_t* out, const uint32
 }
 
 // ---------------------------------------------------------------------------
-// Plain per-gate form, lvl1 API (IKS-BR order), one gate per launch.
-// Binary gates: one job; MUX/NMUX: two jobs run concurrently, then combined
-// (reference src/bootstrap_gpu.cu:1223-1246, :2069-2197).
-template <bool KB, bool MUX>
-__global__ __launch_bounds__(512, 1) void k_gate_lvl1_fft(
-    uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
-    int32_t cb, uint32_t offset, int32_t mux_sign, const uint32_t* ksk,
-    FourierKeys<lvl1param> K)
-{
-    using P = lvl1param;
-    constexpr int C = MUX ? 2 : 1;
-    constexpr int N = P::n, H = N / 2, n0 = lvl0param::n;
-    constexpr uint32_t mu = static_cast<uint32_t>(P::μ);
-    constexpr int NB = BrShape<P>::NB;
-    __shared__ cplx sh_spec[2 * C][NB * H];
-    __shared__ uint32_t sh_tl0[C][kTlwe0Pad];
-    __shared__ uint32_t sh_res[MUX ? 2 : 1][MUX ? N + 1 : 1];
-    __shared__ uint32_t sh_red[8 * (n0 + 1)];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int slot = wave >> 1, j = wave & 1;
-    // key switch over all eight waves of the workgroup (MUX: four per
-    // rotation input), then only the rotation's 2 C waves go on; a
-    // workgroup barrier waits only for the waves that have not ended
-    if constexpr (MUX) {
-        // job 0: c + t - mu ; job 1: -c + f - mu (both AND-like, +-mu out)
-        const int job = wave >> 2;
-        key_switch_waves<TFHEpp::lvl10param, false, 4>(
-            sh_tl0[job], inc, job == 0 ? in1 : in0, job == 0 ? 1 : -1, 1, 0u - mu, ksk,
-            sh_red + job * 4 * (n0 + 1), wave & 3, threadIdx.x & 63);
-    }
-    else {
-        key_switch_waves<TFHEpp::lvl10param, false, 8>(sh_tl0[0], in0, in1, ca, cb, offset, ksk,
-                                                       sh_red, wave, threadIdx.x & 63);
-    }
-    __syncthreads();
-    if (wave >= 2 * C) return;
-    AccStore<P> acc;
-    blind_rotate_fft<P, KB>(sh_tl0[slot], mu, acc, j, sh_spec[wave], sh_spec[wave ^ 1], K);
-    if constexpr (!MUX) {
-        sample_extract_store<P>(acc, j, out);
-    }
-    else {
-        sample_extract_store<P>(acc, j, sh_res[slot]);
-        __syncthreads();
-        for (int i = threadIdx.x; i <= N; i += 256) {
-            uint32_t v = sh_res[0][i] + sh_res[1][i];
-            if (i == N) v += mu;
-            out[i] = mux_sign > 0 ? v : 0u - v;
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Plain per-gate form with the key bundle at lvl1, one gate per workgroup of
-// eight waves on br_fft_pw.hpp's rotation: four transform waves and four that
+// Plain per-gate form at lvl1 (reference src/bootstrap_gpu.cu:1223-1246,
+// :1557-1672, :2069-2197, src/cufhe_gates_gpu.cu:198-511), one gate per
+// workgroup of eight waves on br_fft_pw.hpp's rotation: four transform waves and four that
 // help with the products and the roots (MUX/NMUX: two jobs of four transform
 // waves). Same key switch and rotation as the batched form, so the outputs are
 // the same words. One NAND of the lvl1 API took 3.80 ms with the rotation on a
 // single wave and the others only streaming the key; now 1.23 ms (MUX 4.40 ->
 // 1.84 ms).
-template <bool MUX>
-using GateShape = PwShape<lvl1param, MUX ? 2 : 1, 1, 1, 8, MUX ? 0 : 4>;
+template <bool KB, bool MUX>
+using GateShape = PwShape<lvl1param, MUX ? 2 : 1, 1, 1, 8, MUX ? 0 : 4, KB>;
 
 // coefficient i of SampleExtractIndex<0> of job `job` (its components lie in
 // the digit 0 buffers after rotate())
@@ -353,14 +237,14 @@ __device__ __forceinline__ uint32_t gate_sample(const PwWave<S>& w, int job, int
 }
 
 // lvl1 API (IKS then BR): MUX/NMUX run c + t - mu and -c + f - mu.
-template <bool MUX>
+template <bool KB, bool MUX>
 __global__ __launch_bounds__(512, 2) void k_gate_lvl1_pw(
     uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
     int32_t cb, uint32_t offset, int32_t mux_sign, const uint32_t* ksk,
     FourierKeys<lvl1param> K)
 {
     using P = lvl1param;
-    using S = GateShape<MUX>;
+    using S = GateShape<KB, MUX>;
     static_assert(S::NT == 512, "eight waves");
     constexpr int N = P::n, n0 = lvl0param::n;
     constexpr uint32_t mu = static_cast<uint32_t>(P::μ);
@@ -383,11 +267,8 @@ __global__ __launch_bounds__(512, 2) void k_gate_lvl1_pw(
                                                        red, w.wave, w.lane);
     }
     __syncthreads();
-    const uint32_t* const tl = sh_tl0[w.slot];
-    auto abar = [&](int i) -> uint32_t {
-        return __builtin_amdgcn_readfirstlane(mod_switch<P>(tl[i] + rnd));
-    };
-    w.rotate(true, __builtin_amdgcn_readfirstlane(2 * N - mod_switch<P>(tl[n0])), mu, abar);
+    const PwMask mask{sh_tl0[w.slot], nullptr, 1, 0};
+    w.rotate(true, mask.body<P>(0), mu, mask);
     __syncthreads();
     for (int i = threadIdx.x; i <= N; i += S::NT) {
         uint32_t v = gate_sample(w, 0, i);
@@ -401,14 +282,14 @@ __global__ __launch_bounds__(512, 2) void k_gate_lvl1_pw(
 
 // lvl0 API (BR then IKS): the pre-added lvl0 inputs are mod-switched as they
 // are read; the extracted samples wait in LDS for the key switch.
-template <bool MUX, bool SUBSET>
+template <bool KB, bool MUX, bool SUBSET>
 __global__ __launch_bounds__(512, 2) void k_gate_lvl01_pw(
     uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
     int32_t cb, uint32_t offset, int32_t mux_sign, uint32_t tv_mu, const uint32_t* ksk,
     FourierKeys<lvl1param> K)
 {
     using P = lvl1param;
-    using S = GateShape<MUX>;
+    using S = GateShape<KB, MUX>;
     constexpr int N = P::n, n0 = lvl0param::n;
     constexpr uint32_t mu = static_cast<uint32_t>(P::μ);
     constexpr uint32_t mu0 = static_cast<uint32_t>(lvl0param::μ);
@@ -423,11 +304,8 @@ __global__ __launch_bounds__(512, 2) void k_gate_lvl01_pw(
     const uint32_t sa = static_cast<uint32_t>(MUX ? (w.slot == 0 ? 1 : -1) : ca);
     const uint32_t sb = static_cast<uint32_t>(MUX ? 1 : cb);
     const uint32_t off = MUX ? 0u - mu0 : offset;
-    auto abar = [&](int i) -> uint32_t {
-        return __builtin_amdgcn_readfirstlane(mod_switch<P>(sa * a[i] + sb * b[i] + rnd));
-    };
-    w.rotate(true, __builtin_amdgcn_readfirstlane(2 * N - mod_switch<P>(sa * a[n0] + sb * b[n0] + off)),
-             tv_mu, abar);
+    const PwMask mask{a, b, sa, sb};
+    w.rotate(true, mask.body<P>(off), tv_mu, mask);
     __syncthreads();
 #pragma unroll
     for (int job = 0; job < S::J; job++)
@@ -448,7 +326,7 @@ __global__ __launch_bounds__(512, 2) void k_gate_lvl01_pw(
 // (Torus64), SE, key switch lvl2 -> lvl0 (reference src/bootstrap_gpu.cu
 // :1248-1273, :1305-1331, MUX :1949-2060). MUX runs its two rotations one
 // after the other in the same wave pair (LDS holds one lvl2 job).
-template <bool KB, bool MUX>
+template <bool MUX>
 __global__ __launch_bounds__(256, 1) void k_gate_lvl02_fft(
     uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
     int32_t cb, uint32_t offset, int32_t mux_sign, const uint32_t* ksk,
@@ -490,11 +368,11 @@ __global__ __launch_bounds__(256, 1) void k_gate_lvl02_fft(
         }
         __syncthreads();
         if (rotating) {
-            blind_rotate_fft<P, KB>(sh_tl0, mu, acc, j, sh_spec[j], sh_spec[j ^ 1], K);
+            blind_rotate_fft<P, false>(sh_tl0, mu, acc, j, sh_spec[j], sh_spec[j ^ 1], K);
             sample_extract_store<P>(acc, j, sh_res[pass]);
         }
         else {
-            blind_rotate_ghost<P, KB>(K);
+            blind_rotate_ghost<P, false>(K);
         }
     }
     __syncthreads();
@@ -509,6 +387,68 @@ __global__ __launch_bounds__(256, 1) void k_gate_lvl02_fft(
         key_switch_waves<TFHEpp::lvl20param, false, 4>(out, sh_res[0], nullptr, 1, 0, 0, ksk, red,
                                                        wave, threadIdx.x & 63);
     }
+}
+
+// The same with the key bundle on br_fft_pw.hpp's rotation (eight waves). MUX
+// runs its two rotations one after the other (the LDS holds one lvl2 job); the
+// first one's sample waits in registers.
+template <bool MUX>
+__global__ __launch_bounds__(512, 2) void k_gate_lvl02_pw(
+    uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
+    int32_t cb, uint32_t offset, int32_t mux_sign, const uint32_t* ksk,
+    FourierKeys<lvl2param> K)
+{
+    using P = lvl2param;
+    using T = uint64_t;
+    using S = Lvl2Shape;
+    constexpr int N = P::n, n0 = lvl0param::n, PER = N / S::NT;
+    constexpr T mu = static_cast<T>(P::μ);
+    constexpr uint32_t mu0 = static_cast<uint32_t>(lvl0param::μ);
+    static_assert(S::NT == 512, "eight waves");
+    __shared__ PwShared<S> sm;
+    PwWave<S> w(sm, K, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
+    w.load_tables(threadIdx.x);
+    __syncthreads();
+    T sum[PER + 1];  // coefficients threadIdx.x + 512 k of the sample, then its body
+#pragma unroll
+    for (int k = 0; k <= PER; k++) sum[k] = 0;
+#pragma unroll 1
+    for (int pass = 0; pass < (MUX ? 2 : 1); pass++) {
+        // MUX: pass 0 = c + t - mu, pass 1 = -c + f - mu
+        const uint32_t* a = MUX ? inc : in0;
+        const uint32_t* b = MUX ? (pass == 0 ? in1 : in0) : in1;
+        const uint32_t sa = static_cast<uint32_t>(MUX ? (pass == 0 ? 1 : -1) : ca);
+        const uint32_t sb = static_cast<uint32_t>(MUX ? 1 : cb);
+        const uint32_t off = MUX ? 0u - mu0 : offset;
+        const PwMask mask{a, b, sa, sb};
+        w.rotate(true, mask.body<P>(off), mu, mask);
+        __syncthreads();
+        const T* ca0 = reinterpret_cast<const T*>(w.buf(0, 0, 0));
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int i = threadIdx.x + S::NT * k;
+            sum[k] += i == 0 ? ca0[0] : static_cast<T>(0 - ca0[N - i]);
+        }
+        sum[PER] += reinterpret_cast<const T*>(w.buf(0, 1, 0))[0];
+        __syncthreads();
+    }
+    // key switch of the sum over all eight waves; the sample and the partial
+    // sums lie in transform buffers
+    T* const sample = reinterpret_cast<T*>(w.buf(0, 0, 1));
+    uint32_t* const red = reinterpret_cast<uint32_t*>(w.buf(0, 0, 2));
+    static_assert(sizeof(sm.buf[0]) * 2 >= 8 * (n0 + 1) * 4 && sizeof(sm.buf[0]) >= (N + 1) * sizeof(T),
+                  "buffers");
+#pragma unroll
+    for (int k = 0; k < PER; k++) sample[threadIdx.x + S::NT * k] = sum[k];
+    if (threadIdx.x == 0) sample[N] = sum[PER];
+    __syncthreads();
+    if constexpr (MUX)
+        key_switch_waves<TFHEpp::lvl20param, false, 8>(out, sample, nullptr, mux_sign, 0,
+                                                       mux_sign > 0 ? mu : 0 - mu, ksk, red, w.wave,
+                                                       w.lane);
+    else
+        key_switch_waves<TFHEpp::lvl20param, false, 8>(out, sample, nullptr, 1, 0, 0, ksk, red, w.wave,
+                                                       w.lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -645,7 +585,7 @@ void launch_xai_poly(int32_t* out, hipStream_t st)
 template void launch_xai_poly<lvl1param>(int32_t*, hipStream_t);
 template void launch_xai_poly<lvl2param>(int32_t*, hipStream_t);
 
-// lvl1 key-bundle rotation (br_fft_pw.hpp). c = 1, 2, 4: that many jobs per
+// lvl1 rotation (br_fft_pw.hpp). Key bundle, c = 1, 2, 4: that many jobs per
 // workgroup throughout; else (6, 8, the default) the mix that takes the fewest
 // rounds of the CUs: four jobs per CU share a key pass and the LDS best
 // (2.97 ms a round of 1024 jobs, 11.3 ms for 4096), a CU with two or one is
@@ -653,33 +593,66 @@ template void launch_xai_poly<lvl2param>(int32_t*, hipStream_t);
 // at four and what is left at the smallest width that holds it in one round.
 // Eight-wave workgroups of one wave per job, the form before, took 3.5 / 3.7 /
 // 4.2 / 12.0 ms for 256 / 512 / 1024 / 4096 jobs.
-template <int J, int DPW, int PF, int HELP>
+// CMUX keys (one TRGSW per key bit) add the accumulators to the LDS, so two
+// jobs per workgroup are the most; c = 4 and 8 (the default) mix two and one.
+template <bool KB, int J, int DPW, int PF, int HELP>
 static void launch_pw_lvl1(const BrJob* jobs, int njobs, uint32_t mu,
                            const FourierKeys<lvl1param>& K, hipStream_t st)
 {
-    using S = PwShape<lvl1param, J, 1, DPW, PF, HELP>;
+    using S = PwShape<lvl1param, J, 1, DPW, PF, HELP, KB>;
     if (njobs > 0)
         hipLaunchKernelGGL((k_br_fft_pw<S, 2>), dim3((njobs + J - 1) / J), dim3(S::NT), 0, st, jobs,
                            njobs, mu, K);
 }
-static void launch_br_kb_lvl1(const BrJob* jobs, int njobs, int c, uint32_t mu,
-                              const FourierKeys<lvl1param>& K, hipStream_t st)
+template <bool KB>
+static void launch_br_lvl1(const BrJob* jobs, int njobs, int c, uint32_t mu,
+                           const FourierKeys<lvl1param>& K, hipStream_t st)
 {
+    constexpr int most = KB ? 4 : 2;
     const int cus = device_cu_count();
-    int four = 0;
-    if (c == 4) {
-        four = njobs;
+    int full = 0;  // jobs in workgroups of `most`
+    if (c == most && KB) {
+        full = njobs;
     }
     else if (c != 1 && c != 2) {
-        four = njobs / (4 * cus) * (4 * cus);
-        if (njobs - four > 2 * cus) four = njobs;
+        full = njobs / (most * cus) * (most * cus);
+        if (njobs - full > most / 2 * cus) full = njobs;
     }
-    const int left = njobs - four;
-    launch_pw_lvl1<4, 2, 4, 0>(jobs, four, mu, K, st);
-    if (c == 2 || (c != 1 && left > cus))
-        launch_pw_lvl1<2, 1, 8, 0>(jobs + four, left, mu, K, st);
+    if constexpr (KB)
+        launch_pw_lvl1<true, 4, 2, 4, 0>(jobs, full, mu, K, st);
     else
-        launch_pw_lvl1<1, 1, 8, 4>(jobs + four, left, mu, K, st);
+        launch_pw_lvl1<false, 2, 1, 8, 0>(jobs, full, mu, K, st);
+    const int left = njobs - full;
+    if (c == 2 || (c != 1 && left > cus))
+        launch_pw_lvl1<KB, 2, 1, 8, 0>(jobs + full, left, mu, K, st);
+    else
+        launch_pw_lvl1<KB, 1, 1, 8, 4>(jobs + full, left, mu, K, st);
+}
+
+// lvl2 rotation. Key bundle (c = 1): br_fft_pw.hpp, one job per workgroup and
+// CU; CMUX keys, or c = 2 (a tuning option, two jobs per workgroup): two waves
+// per job. All in a resident grid with a grid stride: the key (167 MB, bundle
+// 250 MB) outgrows the caches once the workgroups drift apart.
+template <bool KB, int C>
+static void launch_br_two_wave(const BrJob* jobs, int njobs, uint64_t mu,
+                               const FourierKeys<lvl2param>& K, hipStream_t st)
+{
+    const int groups = (njobs + C - 1) / C, cap = br_fft_resident_groups<lvl2param, KB, C>();
+    hipLaunchKernelGGL((k_br_fft<lvl2param, KB, C>), dim3(cap > 0 && groups > cap ? cap : groups),
+                       dim3(128 * C), 0, st, jobs, njobs, mu, K);
+}
+template <bool KB>
+static void launch_br_lvl2(const BrJob* jobs, int njobs, int c, uint64_t mu,
+                           const FourierKeys<lvl2param>& K, hipStream_t st)
+{
+    const int cus = device_cu_count();
+    if (c == 2)
+        launch_br_two_wave<KB, 2>(jobs, njobs, mu, K, st);
+    else if constexpr (KB)
+        hipLaunchKernelGGL((k_br_fft_pw<Lvl2Shape, 2>), dim3(njobs < cus ? njobs : cus),
+                           dim3(Lvl2Shape::NT), 0, st, jobs, njobs, mu, K);
+    else
+        launch_br_two_wave<KB, 1>(jobs, njobs, mu, K, st);
 }
 
 template <class P, bool KB>
@@ -687,51 +660,10 @@ void launch_br_fft(const BrJob* jobs, int njobs, int c, typename P::T mu,
                    const FourierKeys<P>& K, hipStream_t st)
 {
     if (njobs <= 0) return;
-    if constexpr (KB && sizeof(typename P::T) == 4) {
-        launch_br_kb_lvl1(jobs, njobs, c, mu, K, st);
-    }
-    else {
-        const dim3 block(128 * c);
-        const dim3 grid((njobs + c - 1) / c);
-        switch (c) {
-            case 1: {
-                // one resident grid (grid-stride over the jobs) for the Torus64
-                // rotation, whose key (167 MB, KB 250 MB) outgrows the caches
-                // once the workgroups drift apart
-                dim3 g1 = grid;
-                if constexpr (sizeof(typename P::T) == 8) {
-                    const int cap = br_fft_resident_groups<P, KB, 1>();
-                    if (cap > 0 && static_cast<int>(g1.x) > cap) g1.x = cap;
-                }
-                hipLaunchKernelGGL((k_br_fft<P, KB, 1>), g1, block, 0, st, jobs, njobs, mu, K);
-                break;
-            }
-            case 2: {
-                // Torus64: two jobs (136 KiB LDS) per workgroup in a resident grid,
-                // their key loads issued together (a tuning option; one job per
-                // workgroup measured faster on the lvl02 mix)
-                dim3 g2 = grid;
-                if constexpr (sizeof(typename P::T) == 8) {
-                    const int cap = br_fft_resident_groups<P, KB, 2>();
-                    if (cap > 0 && static_cast<int>(g2.x) > cap) g2.x = cap;
-                }
-                hipLaunchKernelGGL((k_br_fft<P, KB, 2>), g2, block, 0, st, jobs, njobs, mu, K);
-                break;
-            }
-            case 4:
-                if constexpr (sizeof(typename P::T) == 4)
-                    hipLaunchKernelGGL((k_br_fft<P, KB, 4>), grid, block, 0, st, jobs, njobs, mu,
-                                       K);
-                break;
-            case 8:
-                if constexpr (sizeof(typename P::T) == 4)
-                    hipLaunchKernelGGL((k_br_fft<P, KB, 8>), grid, block, 0, st, jobs, njobs, mu,
-                                       K);
-                break;
-            default:
-                break;
-        }
-    }
+    if constexpr (sizeof(typename P::T) == 4)
+        launch_br_lvl1<KB>(jobs, njobs, c, mu, K, st);
+    else
+        launch_br_lvl2<KB>(jobs, njobs, c, mu, K, st);
 }
 template void launch_br_fft<lvl1param, true>(const BrJob*, int, int, uint32_t,
                                              const FourierKeys<lvl1param>&, hipStream_t);
@@ -747,17 +679,11 @@ void launch_gate_lvl1_fft(bool kb, bool mux, uint32_t* out, const uint32_t* in0,
                           uint32_t offset, int32_t mux_sign, const uint32_t* ksk,
                           const FourierKeys<lvl1param>& K, hipStream_t st)
 {
-    const dim3 grid(1), block(512);
-#define CUFHE_L(KBV, MUXV)                                                                    \
-    hipLaunchKernelGGL((k_gate_lvl1_fft<KBV, MUXV>), grid, block, 0, st, out, in0, in1, inc, \
+#define CUFHE_L(KBV, MUXV)                                                                     \
+    hipLaunchKernelGGL((k_gate_lvl1_pw<KBV, MUXV>), dim3(1), dim3(512), 0, st, out, in0, in1, inc, \
                        ca, cb, offset, mux_sign, ksk, K)
     if (kb) {
-        if (mux)
-            hipLaunchKernelGGL((k_gate_lvl1_pw<true>), grid, dim3(512), 0, st, out, in0, in1, inc,
-                               ca, cb, offset, mux_sign, ksk, K);
-        else
-            hipLaunchKernelGGL((k_gate_lvl1_pw<false>), grid, dim3(512), 0, st, out, in0, in1,
-                               inc, ca, cb, offset, mux_sign, ksk, K);
+        if (mux) CUFHE_L(true, true); else CUFHE_L(true, false);
     }
     else {
         if (mux) CUFHE_L(false, true); else CUFHE_L(false, false);
@@ -770,29 +696,20 @@ void launch_gate_lvl01_fft(bool kb, bool mux, bool subset, uint32_t* out, const 
                            uint32_t offset, int32_t mux_sign, uint32_t tv_mu, const uint32_t* ksk,
                            const FourierKeys<lvl1param>& K, hipStream_t st)
 {
-#define CUFHE_G01(KBV, MUXV, SUB)                                                              \
-    hipLaunchKernelGGL((k_gate_lvl01_fft<KBV, MUXV, SUB>), dim3(1), dim3(512), 0, \
-                       st, out, in0, in1, inc, ca, cb, offset, mux_sign, tv_mu, ksk, K)
-    if (kb) {
-#define CUFHE_K01(MUXV, SUB)                                                                     \
-    hipLaunchKernelGGL((k_gate_lvl01_pw<MUXV, SUB>), dim3(1), dim3(512), 0, st, out, in0, in1, \
+#define CUFHE_G01(KBV, MUXV, SUB)                                                                 \
+    hipLaunchKernelGGL((k_gate_lvl01_pw<KBV, MUXV, SUB>), dim3(1), dim3(512), 0, st, out, in0, in1, \
                        inc, ca, cb, offset, mux_sign, tv_mu, ksk, K)
-        if (mux) {
-            if (subset) CUFHE_K01(true, true); else CUFHE_K01(true, false);
-        }
-        else {
-            if (subset) CUFHE_K01(false, true); else CUFHE_K01(false, false);
-        }
-#undef CUFHE_K01
+#define CUFHE_G01S(KBV, MUXV)                                                      \
+    do {                                                                           \
+        if (subset) CUFHE_G01(KBV, MUXV, true); else CUFHE_G01(KBV, MUXV, false); \
+    } while (0)
+    if (kb) {
+        if (mux) CUFHE_G01S(true, true); else CUFHE_G01S(true, false);
     }
     else {
-        if (mux) {
-            if (subset) CUFHE_G01(false, true, true); else CUFHE_G01(false, true, false);
-        }
-        else {
-            if (subset) CUFHE_G01(false, false, true); else CUFHE_G01(false, false, false);
-        }
+        if (mux) CUFHE_G01S(false, true); else CUFHE_G01S(false, false);
     }
+#undef CUFHE_G01S
 #undef CUFHE_G01
 }
 
@@ -811,15 +728,20 @@ void launch_gate_lvl02_fft(bool kb, bool mux, uint32_t* out, const uint32_t* in0
                            uint32_t offset, int32_t mux_sign, const uint32_t* ksk,
                            const FourierKeys<lvl2param>& K, hipStream_t st)
 {
-    const dim3 grid(1), block(256);
-#define CUFHE_L(KBV, MUXV)                                                                     \
-    hipLaunchKernelGGL((k_gate_lvl02_fft<KBV, MUXV>), grid, block, 0, st, out, in0, in1, inc, \
-                       ca, cb, offset, mux_sign, ksk, K)
+    const dim3 grid(1);
+#define CUFHE_L(MUXV)                                                                          \
+    hipLaunchKernelGGL((k_gate_lvl02_fft<MUXV>), grid, dim3(256), 0, st, out, in0, in1, inc, ca, \
+                       cb, offset, mux_sign, ksk, K)
     if (kb) {
-        if (mux) CUFHE_L(true, true); else CUFHE_L(true, false);
+        if (mux)
+            hipLaunchKernelGGL((k_gate_lvl02_pw<true>), grid, dim3(512), 0, st, out, in0, in1, inc, ca,
+                               cb, offset, mux_sign, ksk, K);
+        else
+            hipLaunchKernelGGL((k_gate_lvl02_pw<false>), grid, dim3(512), 0, st, out, in0, in1, inc, ca,
+                               cb, offset, mux_sign, ksk, K);
     }
     else {
-        if (mux) CUFHE_L(false, true); else CUFHE_L(false, false);
+        if (mux) CUFHE_L(true); else CUFHE_L(false);
     }
 #undef CUFHE_L
 }

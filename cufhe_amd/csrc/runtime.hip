@@ -897,13 +897,10 @@ int lvl1_pick_c(int c, int nbr)
             // the ring's barriers
             c = 2;
         }
-        else if (k.kb) {
-            // the mix of workgroup widths that launch_br_kb_lvl1 picks by the
+        else {
+            // the mix of workgroup widths that launch_br_lvl1 picks by the
             // number of jobs
             c = 8;
-        }
-        else {
-            c = 1;
         }
     }
     // 6: the NTT kernels that share key chunks among six jobs through LDS; with

@@ -1,5 +1,6 @@
-"""The key-bundle rotation at the edges of its workgroup widths: counts that fill
-no workgroup, exactly one round, or one job more (FFT backend, lvl1)."""
+"""The lvl1 rotations at the edges of their workgroup widths: counts that fill
+no workgroup, exactly one round, or one job more (FFT backend, key bundle and
+CMUX keys); the lvl2 key-bundle rotation against the two-wave kernel."""
 import numpy as np
 import pytest
 
@@ -10,19 +11,21 @@ from conftest import load_lvl1_keys
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module")
-def rotations(keys_lvl1):
+@pytest.fixture(scope="module", params=[True, False], ids=["bundle", "cmux"])
+def rotations(request, keys_lvl1):
     """1027 random lvl0 samples, some with masks that round to 0, N and 2N - 1,
     and their rotations by the one-job workgroups."""
+    kb = request.param
     C.check(C.lib().cufhe_initialize(), "initialize")
-    load_lvl1_keys(("fft", True), keys_lvl1["bk_kb"], keys_lvl1["ksk"],
-                   backend=C.BACKEND_FFT, variant=C.BR_KEY_BUNDLE)
+    bk = keys_lvl1["bk_kb" if kb else "bk"]
+    load_lvl1_keys(("fft", kb), bk, keys_lvl1["ksk"], backend=C.BACKEND_FFT,
+                   variant=C.BR_KEY_BUNDLE if kb else C.BR_PLAIN)
     rng = np.random.default_rng(61)
     tl0 = rng.integers(0, 2**32, (1027, 637), dtype=np.uint64).astype(np.uint32)
     tl0[0] = 0
     tl0[1] = np.uint32(1 << 31)
     tl0[2] = np.uint32(0xFFFFFFFF)
-    return tl0, _run(tl0, 1)
+    return kb, bk, tl0, _run(tl0, 1)
 
 
 def _run(tl0, c):
@@ -32,16 +35,39 @@ def _run(tl0, c):
     return dout.download(np.uint32, (tl0.shape[0], C.TLWE1_WORDS))
 
 
-def test_one_job_workgroups_equal_the_exact_oracle(rotations, keys_lvl1):
+def test_one_job_workgroups_equal_the_exact_oracle(rotations):
     # integers: the FP64 product is within a small fraction of a unit of them
-    tl0, out = rotations
+    kb, bk, tl0, out = rotations
     for i in (0, 1, 2, 3, 1026):
-        acc = O.blind_rotate(1, O.EXACT, True, tl0[i], keys_lvl1["bk_kb"], C.MU1)
+        acc = O.blind_rotate(1, O.EXACT, kb, tl0[i], bk, C.MU1)
         assert np.array_equal(out[i], O.sample_extract(1, acc)), i
 
 
 @pytest.mark.parametrize("c", [0, 2, 4])
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 255, 256, 257, 512, 513, 1024, 1027])
 def test_widths_agree(rotations, c, n):
-    tl0, out = rotations
+    _, _, tl0, out = rotations
     assert np.array_equal(_run(tl0[:n], c), out[:n])
+
+
+def test_lvl2_bundle_equals_the_two_wave_kernel(keys_lvl2):
+    """Every bit: both forms do the same operations in the same order."""
+    C.check(C.lib().cufhe_initialize(), "initialize")
+    C.initialize_lvl02(keys_lvl2["bk_kb"], keys_lvl2["ksk"])
+    rng = np.random.default_rng(62)
+    n = 259  # a job more than the CUs, and an odd one for the two-job groups
+    tl0 = rng.integers(0, 2**32, (n, 637), dtype=np.uint64).astype(np.uint32)
+    tl0[0] = 0
+    tl0[1] = np.uint32(1 << 31)
+    tl0[2] = np.uint32(0xFFFFFFFF)
+    din = C.DeviceBuffer.from_numpy(tl0)
+    out = {}
+    try:
+        for c in (1, 2):
+            C.check(C.lib().cufhe_set_lvl2_jobs_per_group(c), "jobs per group")
+            dout = C.DeviceBuffer(n * C.TLWE2_WORDS * 8)
+            C.check(C.lib().cufhe_bootstrap_lvl02(dout.ptr, din.ptr, C.MU2, n, None), "bootstrap")
+            out[c] = dout.download(np.uint64, (n, C.TLWE2_WORDS))
+    finally:
+        C.check(C.lib().cufhe_set_lvl2_jobs_per_group(1), "jobs per group")
+    assert np.array_equal(out[1], out[2])
