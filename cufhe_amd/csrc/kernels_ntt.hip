@@ -2,17 +2,15 @@
 // rotation (plain CMUX, key bundle, block-binary), the plain per-gate form,
 // and transform entry points for the parity tests.
 #include "br_ntt.hpp"
-#include "br_ntt_shared.hpp"
+#include "br_ntt_pw.hpp"
 #include "keyswitch.hpp"
 #include "launch.hpp"
+
+#include <algorithm>
 
 namespace cufhe_amd {
 
 constexpr int kNttTlwe0Pad = 640;  // lvl0 TLWE (637 words) padded in LDS
-
-#ifndef CUFHE_BR_NTT_WAVES_PER_SIMD
-#define CUFHE_BR_NTT_WAVES_PER_SIMD 3
-#endif
 
 // ---------------------------------------------------------------------------
 // Torus32 polynomials -> NTT spectra in Montgomery form, one wave per
@@ -75,50 +73,20 @@ __global__ __launch_bounds__(256) void k_ntt_natural(uint32_t* out, const uint32
 }
 
 // ---------------------------------------------------------------------------
-// Batched blind rotation + SampleExtract: C jobs per workgroup, two waves per
-// job (wave j owns TRLWE component j). Inputs are pre-added lvl0 TLWEs.
-template <int MODE, int C>
-__global__ __launch_bounds__(128 * C, CUFHE_BR_NTT_WAVES_PER_SIMD) void k_br_ntt(
-    const BrJob* __restrict__ jobs, int njobs, uint32_t mu, NttKeys K)
-{
-    constexpr int n0 = lvl0param::n;
-    __shared__ uint32_t sh_lds[2 * C][kNttLdsWords];
-    __shared__ uint32_t sh_tl0[C][kNttTlwe0Pad];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int slot = wave >> 1, j = wave & 1;
-    const int raw = blockIdx.x * C + slot;
-    const bool live = raw < njobs;
-    const BrJob jb = jobs[live ? raw : njobs - 1];
-    for (int i = threadIdx.x & 127; i <= n0; i += 128) {
-        uint32_t v = static_cast<uint32_t>(jb.ca) * jb.in0[i];
-        if (jb.in1) v += static_cast<uint32_t>(jb.cb) * jb.in1[i];
-        if (i == n0) v += jb.offset;
-        sh_tl0[slot][i] = v;
-    }
-    __syncthreads();
-    uint32_t acc[16];
-    blind_rotate_ntt<MODE>(sh_tl0[slot], mu, acc, j, sh_lds[wave], sh_lds[wave ^ 1], K);
-    if (live) {
-        if (jb.flags & kBrOutTrlwe)
-            trlwe_store_ntt(acc, j, static_cast<uint32_t*>(jb.out));
-        else
-            sample_extract_ntt(acc, j, static_cast<uint32_t*>(jb.out));
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Batched rotation with the key shared by the workgroup's C jobs through an
-// LDS ring (br_ntt_shared.hpp); one workgroup of 2C waves per CU.
-template <int MODE, int C>
-__global__ __launch_bounds__(128 * C, 1) void k_br_ntt_shared(const BrJob* __restrict__ jobs,
-                                                               int njobs, uint32_t mu, NttKeys K)
+// Batched blind rotation + SampleExtract, up to kNttPwJobs jobs per workgroup
+// (the jobs spread evenly, the larger shares first) with the products split over
+// all its waves by bins (br_ntt_pw.hpp); one workgroup of sixteen waves per CU.
+// Inputs are pre-added lvl0 TLWEs; wave 2 s + j rotates component j of job s.
+template <int MODE>
+__global__ __launch_bounds__(kNttPwThreads, 1) void k_br_ntt_pw(const BrJob* __restrict__ jobs,
+                                                                int njobs, uint32_t mu, NttKeys K)
 {
     using P = lvl1param;
     constexpr int N = P::n, n0 = lvl0param::n;
-    constexpr int NT = 128 * C;
+    constexpr int NT = kNttPwThreads;
     constexpr uint32_t rnd = kMaskRound<P>;
     constexpr int shift = 32 - 1 - P::nbit;
-    __shared__ NttShared<C> sm;
+    __shared__ NttPwShared sm;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = wave >> 1, j = wave & 1;
     const int t = threadIdx.x;
@@ -134,30 +102,38 @@ __global__ __launch_bounds__(128 * C, 1) void k_br_ntt_shared(const BrJob* __res
         sm.cr[i] = K.tb.cr[i];
         sm.cri[i] = K.tb.cri[i];
     }
-    for (int i = t; i < 2 * N; i += NT) sm.pw[i] = K.tb.pw[i];
-    const int raw = blockIdx.x * C + slot;
-    const bool live = raw < njobs;
-    const BrJob jb = jobs[live ? raw : njobs - 1];
-    uint32_t part = 0;
-    for (int i = t & 127; i <= n0; i += 128) {
-        uint32_t v = static_cast<uint32_t>(jb.ca) * jb.in0[i];
-        if (jb.in1) v += static_cast<uint32_t>(jb.cb) * jb.in1[i];
-        if (i < n0) {
-            const uint32_t m = mod_switch<P>(v + rnd);
-            sm.abar[slot][i] = static_cast<uint16_t>(m);
-            part += v - (m << shift);
-        }
-        else {
-            sm.bar[slot] = v + jb.offset;  // body; turned into bar below
-        }
+    for (int i = t; i < 2 * N; i += NT) {
+        const uint32_t v = mod_sub(K.tb.pw[i], ntt31::R1);
+        sm.root[i] = static_cast<int32_t>(v > ntt31::HALF_P ? v - ntt31::P : v);
     }
-    if constexpr (MODE == NTT_BB) {
+    const int group = blockIdx.x, groups = gridDim.x;
+    const int share = njobs / groups, larger = njobs - share * groups;
+    const int first = group * share + min(group, larger);
+    const int live = share + (group < larger ? 1 : 0);  // 1 .. kNttPwJobs
+    const bool rotating = slot < live;
+    const BrJob jb = jobs[rotating ? first + slot : first];
+    if (rotating) {
+        uint32_t part = 0;
+        for (int i = t & 127; i <= n0; i += 128) {
+            uint32_t v = static_cast<uint32_t>(jb.ca) * jb.in0[i];
+            if (jb.in1) v += static_cast<uint32_t>(jb.cb) * jb.in1[i];
+            if (i < n0) {
+                const uint32_t m = mod_switch<P>(v + rnd);
+                sm.abar[slot][i] = static_cast<uint16_t>(m);
+                part += v - (m << shift);
+            }
+            else {
+                sm.bar[slot] = v + jb.offset;  // body; turned into bar below
+            }
+        }
+        if constexpr (MODE == NTT_BB) {
 #pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) part += __shfl_xor(part, m);
-        if ((t & 63) == 0) sm.corr[slot][j] = part;
+            for (int m = 32; m >= 1; m >>= 1) part += __shfl_xor(part, m);
+            if ((t & 63) == 0) sm.corr[slot][j] = part;
+        }
     }
     __syncthreads();
-    if ((t & 127) == 0) {
+    if (rotating && (t & 127) == 0) {
         uint32_t body = sm.bar[slot];
         if constexpr (MODE == NTT_BB) {
             // reference gatebootstrapping_gpu.cuh:814-838
@@ -168,8 +144,8 @@ __global__ __launch_bounds__(128 * C, 1) void k_br_ntt_shared(const BrJob* __res
     }
     __syncthreads();
     uint32_t acc[16];
-    blind_rotate_ntt_shared<MODE, C>(sm, slot, j, mu, acc, K);
-    if (live) {
+    blind_rotate_ntt_pw<MODE>(sm, live, slot, j, mu, acc, K);
+    if (rotating) {
         if (jb.flags & kBrOutTrlwe)
             trlwe_store_ntt(acc, j, static_cast<uint32_t*>(jb.out));
         else
@@ -331,44 +307,23 @@ void launch_ntt_natural(bool inverse, uint32_t* out, const uint32_t* in, int npo
                            npolys, tb);
 }
 
-template <int MODE>
-static void launch_br_ntt_mode(const BrJob* jobs, int njobs, int c, uint32_t mu, const NttKeys& K,
-                               hipStream_t st)
-{
-    if (njobs <= 0) return;
-    switch (c) {
-        case 2:
-            hipLaunchKernelGGL((k_br_ntt<MODE, 2>), dim3((njobs + 1) / 2), dim3(256), 0, st, jobs,
-                               njobs, mu, K);
-            break;
-        case 4:
-            hipLaunchKernelGGL((k_br_ntt<MODE, 4>), dim3((njobs + 3) / 4), dim3(512), 0, st, jobs,
-                               njobs, mu, K);
-            break;
-        case 8:
-            hipLaunchKernelGGL((k_br_ntt<MODE, 8>), dim3((njobs + 7) / 8), dim3(1024), 0, st, jobs,
-                               njobs, mu, K);
-            break;
-        case 6:
-            hipLaunchKernelGGL((k_br_ntt_shared<MODE, 6>), dim3((njobs + 5) / 6), dim3(768), 0, st,
-                               jobs, njobs, mu, K);
-            break;
-        default:
-            hipLaunchKernelGGL((k_br_ntt<MODE, 1>), dim3(njobs), dim3(128), 0, st, jobs, njobs, mu,
-                               K);
-            break;
-    }
-}
-
-void launch_br_ntt(int mode, const BrJob* jobs, int njobs, int c, uint32_t mu, const NttKeys& K,
+// A CU holds one workgroup: the fewest rounds of workgroups with at most `width`
+// jobs each, the jobs spread evenly over them. Block-binary rotations take, with
+// 1, 2, 4, 6 and 8 jobs a CU, 1.5, 1.7, 2.5, 3.5 and 4.5 ms: 8 jobs in one round
+// beat two rounds of 4, and 9 as 5 and 4 beat 8 and 1.
+void launch_br_ntt(int mode, const BrJob* jobs, int njobs, int width, uint32_t mu, const NttKeys& K,
                    hipStream_t st)
 {
+    if (njobs <= 0) return;
+    const int per_round = std::min(width, kNttPwJobs) * device_cu_count();
+    const int rounds = (njobs + per_round - 1) / per_round;
+    const dim3 grid(std::min(njobs, rounds * device_cu_count())), block(kNttPwThreads);
     if (mode == NTT_KB)
-        launch_br_ntt_mode<NTT_KB>(jobs, njobs, c, mu, K, st);
+        hipLaunchKernelGGL(k_br_ntt_pw<NTT_KB>, grid, block, 0, st, jobs, njobs, mu, K);
     else if (mode == NTT_BB)
-        launch_br_ntt_mode<NTT_BB>(jobs, njobs, c, mu, K, st);
+        hipLaunchKernelGGL(k_br_ntt_pw<NTT_BB>, grid, block, 0, st, jobs, njobs, mu, K);
     else
-        launch_br_ntt_mode<NTT_PLAIN>(jobs, njobs, c, mu, K, st);
+        hipLaunchKernelGGL(k_br_ntt_pw<NTT_PLAIN>, grid, block, 0, st, jobs, njobs, mu, K);
 }
 
 template <int MODE, bool SUBSET>

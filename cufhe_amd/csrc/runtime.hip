@@ -890,21 +890,11 @@ int lvl1_pick_c(int c, int nbr)
 {
     const LevelKeys<lvl1param>& k = state().k1;
     if (c == 0) c = tuned_c(nbr);
-    if (c == 0) {
-        if (k.backend == CUFHE_BACKEND_NTT) {
-            // NTT block-binary sweep (4096 gates, BR ms): C=1 18.1, 2 17.3,
-            // 4 20.3, 6 (shared key) 21.6 -- the 4-byte NTT key is not worth
-            // the ring's barriers
-            c = 2;
-        }
-        else {
-            // the mix of workgroup widths that launch_br_lvl1 picks by the
-            // number of jobs
-            c = 8;
-        }
-    }
-    // 6: the NTT kernels that share key chunks among six jobs through LDS; with
-    // the FFT key bundle 6 and 8 are the mix
+    // the widest: the FFT launchers mix workgroup widths by the number of jobs,
+    // the NTT one spreads the jobs evenly over the rounds
+    if (c == 0) c = 8;
+    // with the FFT key bundle 6 and 8 are the mix; NTT: at most c jobs a
+    // workgroup
     if (c == 6) return (k.backend == CUFHE_BACKEND_NTT || k.kb) ? 6 : -1;
     if (c != 1 && c != 2 && c != 4 && c != 8) return -1;
     return c;
