@@ -1,4 +1,6 @@
-// Blind rotation in the Fourier domain (FP64 FFNT backend).
+// Blind rotation in the Fourier domain (FP64 FFNT backend), two waves per job:
+// lvl2 CMUX keys, two lvl2 jobs per workgroup, and the single external product
+// (CMUX). Its step is also the definition that br_fft_pw.hpp keeps to.
 //
 // Reference: include/gatebootstrapping_gpu.cuh:69-221 (Accumulate, CMUX
 // form: acc += ExtProd((X^a - 1) acc, BK_i)), :895-1033 (AccumulateKeyBundle:

@@ -25,8 +25,10 @@
 //     With CMUX keys it adds to the accumulator it keeps and publishes that in
 //     LDS, where phase 1 reads it rotated.
 // What bounds it: FP64 issue and LDS traffic, about equally, over the whole
-// CU. (An LDS KiB costs a CU 5.7 ns written and 3.2 ns read, a wave's FP64
-// instruction 0.5 ns; FP64 MFMA runs on the same pipe as the vector FMAs.)
+// CU. (An LDS KiB costs a CU 5.7 ns written and 3.2 ns read at two waves per
+// SIMD, a wave's FP64 instruction 0.5 ns; FP64 MFMA runs on the same pipe as
+// the vector FMAs.) At lvl2 phase 2 moves 786 KB of key a step at the 46
+// B/cycle that a CU's vector loads reach, and is bound by them.
 #pragma once
 
 #include "br_fft.hpp"
@@ -487,9 +489,11 @@ struct PwWave {
                         for (int m = 0; m < 3; m++) xx[m].x -= 1.0;
                     }
                 };
-                if constexpr (S::kBase) make_x();
+                // with helper waves after the barrier: before it, their key
+                // loads were waited for there (one gate 1.35 against 1.25 ms)
+                if constexpr (S::kBase && !S::HELP) make_x();
                 __syncthreads();  // digit spectra are in LDS
-                if constexpr (S::kTail) make_x();
+                if constexpr (S::kTail || (S::kBase && S::HELP)) make_x();
                 // the spectra of a (digit, component) are loaded while the one
                 // before it is multiplied
                 constexpr int DN = S::BPL * S::QD * 2;

@@ -154,7 +154,7 @@ __global__ __launch_bounds__(kNttPwThreads, 1) void k_br_ntt_pw(const BrJob* __r
 }
 
 // ---------------------------------------------------------------------------
-// Plain per-gate form, lvl0 API (BR-IKS at lvl1), as k_gate_lvl01_fft.
+// Plain per-gate form, lvl0 API (BR-IKS at lvl1), as k_gate_lvl01_pw.
 template <int MODE, bool SUBSET, bool MUX>
 __global__ __launch_bounds__(512, 1) void k_gate_lvl01_ntt(
     uint32_t* out, const uint32_t* in0, const uint32_t* in1, const uint32_t* inc, int32_t ca,
