@@ -1849,7 +1849,6 @@ int cufhe_autotune_lvl1(int nbootstraps, int* best, float* times_ms, void* strea
     float bestt = 0.f;
     for (int c : {1, 2, 4, 6, 8}) {
         if (lvl1_pick_c(c, n) != c) continue;  // not valid for these keys
-        if (c == 8 && !s.k1.kb) continue;
         float t = 0.f;
         for (int rep = 0; rep < 2; rep++) {  // the first launch warms up
             CUFHE_HIP_TRY(hipEventRecord(mem.e[0], st));
