@@ -62,9 +62,9 @@ FP64_PEAK_TFLOPS = 78.6
 HBM_PEAK_GBPS = 8000.0
 # one 64-lane VALU instruction per CU-cycle: 256 CUs x 2.4 GHz
 VALU_PEAK_GINST = 256 * 2.4
-# VALU wave-instructions of one 4096-gate k_br_ntt<2, 2> launch (rocprofv3
-# SQ_INSTS_VALU, profiles/br_ntt_bb_lvl1_batch4096_counters.md)
-NTT_BB_VALU_INSTS_C2 = 7.609e9
+# VALU wave-instructions of one 4096-gate k_br_ntt_pw<2> launch, eight jobs per
+# workgroup (rocprofv3 SQ_INSTS_VALU, profiles/rotations_trace_and_counters.md)
+NTT_BB_VALU_INSTS_C8 = 4.824e9
 # VALU wave-instructions per lvl2 key-bundle bootstrap of k_br_ntt64<true>
 # (rocprofv3 SQ_INSTS_VALU over a 2560-rotation launch,
 # profiles/br_ntt64_kb_lvl2_mix2048_counters.md)
@@ -546,7 +546,7 @@ def workload_nttbb(args):
     br_avg_s = statistics.mean(br_ms) / 1e3
     groups = -(-nbr // best_c)
     key_gbps = BK_BYTES_NTT_BB * groups / br_avg_s / 1e9
-    valu_g = (NTT_BB_VALU_INSTS_C2 / br_avg_s / 1e9) if best_c == 2 else float("nan")
+    valu_g = (NTT_BB_VALU_INSTS_C8 / br_avg_s / 1e9) if best_c == 8 else float("nan")
     res = base_result(args, value, total * 1e3 / args.steps, "u32 mod P", {
         "workload": "batched lvl1 NAND/XOR gates, NTT backend (P=2147473409), block-binary "
                     "lvl0 key (blocks of 4), subset key switching, 4096 gates",
@@ -572,7 +572,7 @@ def workload_nttbb(args):
                                              "alpha_bk=2^-24.8, 8 key-noise terms per block (cufhe_amd/noise.py)"},
         "bit_exact_sample": bit_exact,
         # integer-only kernel bound by VALU issue: VALU wave-instructions per
-        # launch (profiles/br_ntt_bb_lvl1_batch4096_counters.md, C=2) over
+        # launch (profiles/rotations_trace_and_counters.md, C=8) over
         # the live launch time, against one wave-instruction per CU-cycle
         "roofline": {"bound": "valu", "achieved": round(valu_g, 1), "peak": VALU_PEAK_GINST,
                      "unit": "G wave-instr/s", "frac": round(valu_g / VALU_PEAK_GINST, 4),
