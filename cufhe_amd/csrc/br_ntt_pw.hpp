@@ -35,6 +35,7 @@
 #pragma once
 
 #include "br_ntt.hpp"
+#include "launch_rules.hpp"
 
 namespace cufhe_amd {
 
@@ -46,8 +47,7 @@ struct NttModeShape {
     static constexpr int STEPS = lvl0param::n / STEP_BITS;
 };
 
-// Jobs that a workgroup has room for: two waves each, sixteen rows of bins.
-constexpr int kNttPwJobs = 8;
+// two waves a job, sixteen rows of bins
 constexpr int kNttPwThreads = 128 * kNttPwJobs;
 
 struct NttPwShared {

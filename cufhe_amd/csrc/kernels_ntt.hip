@@ -6,8 +6,6 @@
 #include "keyswitch.hpp"
 #include "launch.hpp"
 
-#include <algorithm>
-
 namespace cufhe_amd {
 
 constexpr int kNttTlwe0Pad = 640;  // lvl0 TLWE (637 words) padded in LDS
@@ -307,17 +305,11 @@ void launch_ntt_natural(bool inverse, uint32_t* out, const uint32_t* in, int npo
                            npolys, tb);
 }
 
-// A CU holds one workgroup: the fewest rounds of workgroups with at most `width`
-// jobs each, the jobs spread evenly over them. Block-binary rotations take, with
-// 1, 2, 4, 6 and 8 jobs a CU, 1.5, 1.7, 2.5, 3.5 and 4.5 ms: 8 jobs in one round
-// beat two rounds of 4, and 9 as 5 and 4 beat 8 and 1.
-void launch_br_ntt(int mode, const BrJob* jobs, int njobs, int width, uint32_t mu, const NttKeys& K,
+void launch_br_ntt(int mode, const BrJob* jobs, int njobs, uint32_t mu, const NttKeys& K,
                    hipStream_t st)
 {
     if (njobs <= 0) return;
-    const int per_round = std::min(width, kNttPwJobs) * device_cu_count();
-    const int rounds = (njobs + per_round - 1) / per_round;
-    const dim3 grid(std::min(njobs, rounds * device_cu_count())), block(kNttPwThreads);
+    const dim3 grid(ntt_workgroups(njobs, device_cu_count())), block(kNttPwThreads);
     if (mode == NTT_KB)
         hipLaunchKernelGGL(k_br_ntt_pw<NTT_KB>, grid, block, 0, st, jobs, njobs, mu, K);
     else if (mode == NTT_BB)

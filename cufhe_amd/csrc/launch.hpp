@@ -73,7 +73,7 @@ void launch_to_ntt(uint32_t* out, const uint32_t* in, int npolys, const NttTable
                    hipStream_t st);
 void launch_ntt_natural(bool inverse, uint32_t* out, const uint32_t* in, int npolys,
                         const NttTables& tb, hipStream_t st);
-void launch_br_ntt(int mode, const BrJob* jobs, int njobs, int c, uint32_t mu, const NttKeys& K,
+void launch_br_ntt(int mode, const BrJob* jobs, int njobs, uint32_t mu, const NttKeys& K,
                    hipStream_t st);
 void launch_gate_lvl01_ntt(int mode, bool subset, bool mux, uint32_t* out, const uint32_t* in0,
                            const uint32_t* in1, const uint32_t* inc, int32_t ca, int32_t cb,

@@ -712,7 +712,7 @@ void br_lvl1(const BrJob* jobs, int n, int c, uint32_t mu, hipStream_t st)
     const LevelKeys<lvl1param>& k = state().k1;
     if (n <= 0) return;
     if (k.backend == CUFHE_BACKEND_NTT)
-        launch_br_ntt(k.variant, jobs, n, c, mu, k.nk, st);
+        launch_br_ntt(k.variant, jobs, n, mu, k.nk, st);
     else if (k.kb)
         launch_br_fft<lvl1param, true>(jobs, n, c, mu, k.fk, st);
     else
@@ -890,11 +890,10 @@ int lvl1_pick_c(int c, int nbr)
 {
     const LevelKeys<lvl1param>& k = state().k1;
     if (c == 0) c = tuned_c(nbr);
-    // the widest: the FFT launchers mix workgroup widths by the number of jobs,
-    // the NTT one spreads the jobs evenly over the rounds
+    // the FFT launchers mix workgroup widths by the number of jobs; the NTT one
+    // spreads the jobs evenly over the fewest rounds, whatever c
     if (c == 0) c = 8;
-    // with the FFT key bundle 6 and 8 are the mix; NTT: at most c jobs a
-    // workgroup
+    // with the FFT key bundle 6 and 8 are the mix
     if (c == 6) return (k.backend == CUFHE_BACKEND_NTT || k.kb) ? 6 : -1;
     if (c != 1 && c != 2 && c != 4 && c != 8) return -1;
     return c;

@@ -186,8 +186,8 @@ int cufhe_gate_lvl02(int op, uint32_t* out, const uint32_t* in0, const uint32_t*
  * d_pool + 1025 w). Outputs of a batch must not be read by the same batch.
  * jobs_per_group: bootstraps per workgroup (1, 2, 4, 6, 8; 0 = default).
  * With the FFT key-bundle keys, 6 and 8 (the default) mix workgroups of four,
- * two and one jobs by the size of the batch; with the NTT keys, 6 is the
- * shared-key NTT kernel. use_graph != 0 captures the launches in a HIP graph
+ * two and one jobs by the size of the batch; with the NTT keys every value is
+ * the same launch. use_graph != 0 captures the launches in a HIP graph
  * on the first run and replays it. */
 int cufhe_plan_create_lvl1(const cufhe_gate_desc* gates, int n, uint32_t* d_pool,
                            int jobs_per_group, int use_graph, cufhe_plan** plan);
@@ -212,8 +212,7 @@ int cufhe_plan_jobs_per_group(const cufhe_plan* plan);
 int cufhe_plan_run_timed(cufhe_plan* plan, void* stream, float* kernel_ms);
 /* Autotuner of the batched rotation, no reference counterpart: times every
  * rotation kernel / jobs-per-workgroup choice c valid for the loaded lvl1
- * keys (1, 2, 4; 6: NTT key chunks shared by six jobs through LDS; with the
- * FFT key bundle 6 and 8 mix the widths by batch size) on
+ * keys (the values of jobs_per_group) on
  * nbootstraps synthetic jobs and records the fastest for that batch size.
  * Plans, one-shot batches and servers created with jobs_per_group 0 then use
  * the recorded choice of the smallest tuned size >= their batch (else the

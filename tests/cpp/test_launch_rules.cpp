@@ -1,0 +1,36 @@
+// The launch rules of the lvl1 rotations on the host, for every batch size up to
+// twelve thousand and several CU counts. Runs without a GPU.
+#include "../../cufhe_amd/csrc/launch_rules.hpp"
+
+#include <cstdio>
+#include <cstdlib>
+
+using namespace cufhe_amd;
+
+static long checked = 0;
+static void require(bool ok, const char* what, int njobs, int cus)
+{
+    if (!ok) {
+        std::printf("%s: %d jobs on %d CUs\n", what, njobs, cus);
+        std::exit(1);
+    }
+    checked++;
+}
+static int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// every workgroup has 1 .. 8 jobs, in as few rounds of workgroups as eight jobs take
+static void check_ntt(int njobs, int cus)
+{
+    const int groups = ntt_workgroups(njobs, cus);
+    require(groups >= 1 && groups <= njobs, "empty workgroups", njobs, cus);
+    require(ceil_div(njobs, groups) <= kNttPwJobs, "more than eight jobs", njobs, cus);
+    require(ceil_div(groups, cus) == ceil_div(njobs, kNttPwJobs * cus), "rounds", njobs, cus);
+}
+
+int main()
+{
+    for (int cus : {1, 32, 80, 256, 304})
+        for (int njobs = 1; njobs <= 12000; njobs++) check_ntt(njobs, cus);
+    std::printf("ok: %ld checks\n", checked);
+    return 0;
+}

@@ -1,6 +1,7 @@
 """The NTT-backend rotation at the edges of its shares of jobs: counts that leave
-CUs idle, fill rounds exactly, or make shares of two sizes; every word against
-the one-job workgroups, and those against the oracle."""
+CUs idle, fill rounds exactly, or make shares of two sizes, with every
+jobs_per_group; every word against workgroups of one job, and those against the
+oracle."""
 import numpy as np
 import pytest
 
@@ -13,6 +14,9 @@ pytestmark = pytest.mark.gpu
 MODES = {"plain": (C.BR_PLAIN, O.BR_PLAIN), "kb": (C.BR_KEY_BUNDLE, O.BR_KB),
          "bb": (C.BR_BLOCK_BINARY, O.BR_BB)}
 MOST = 2305
+
+
+ALONE = 100  # jobs of a batch whose workgroups have one job each
 
 
 def _run(tl0, c):
@@ -36,7 +40,8 @@ def rotations(request, keys_lvl1, keys_bb):
     tl0[0] = 0
     tl0[1] = np.uint32(1 << 31)
     tl0[2] = np.uint32(0xFFFFFFFF)
-    return mode, bk, tl0, _run(tl0, 1)
+    alone = [_run(tl0[i:i + ALONE], 1) for i in range(0, MOST, ALONE)]
+    return mode, bk, tl0, np.concatenate(alone)
 
 
 def test_one_job_workgroups_equal_the_oracle(rotations):
@@ -46,7 +51,7 @@ def test_one_job_workgroups_equal_the_oracle(rotations):
         assert np.array_equal(out[i], O.sample_extract(1, acc)), i
 
 
-@pytest.mark.parametrize("c", [0, 2, 6])
+@pytest.mark.parametrize("c", [0, 1, 2, 6])
 @pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 511, 513, 2047, 2048, 2049, MOST])
 def test_shares_agree(rotations, c, n):
     _, _, tl0, out = rotations
