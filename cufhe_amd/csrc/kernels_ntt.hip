@@ -309,7 +309,7 @@ void launch_br_ntt(int mode, const BrJob* jobs, int njobs, uint32_t mu, const Nt
                    hipStream_t st)
 {
     if (njobs <= 0) return;
-    const dim3 grid(ntt_workgroups(njobs, device_cu_count())), block(kNttPwThreads);
+    const dim3 grid(ntt_workgroups(mode == NTT_PLAIN, njobs, device_cu_count())), block(kNttPwThreads);
     if (mode == NTT_KB)
         hipLaunchKernelGGL(k_br_ntt_pw<NTT_KB>, grid, block, 0, st, jobs, njobs, mu, K);
     else if (mode == NTT_BB)
