@@ -4,6 +4,7 @@
 #include "br_fft_pw.hpp"
 #include "keyswitch.hpp"
 #include "launch.hpp"
+#include "launch_rules.hpp"
 
 namespace cufhe_amd {
 
@@ -585,16 +586,7 @@ void launch_xai_poly(int32_t* out, hipStream_t st)
 template void launch_xai_poly<lvl1param>(int32_t*, hipStream_t);
 template void launch_xai_poly<lvl2param>(int32_t*, hipStream_t);
 
-// lvl1 rotation (br_fft_pw.hpp). Key bundle, c = 1, 2, 4: that many jobs per
-// workgroup throughout; else (6, 8, the default) the mix that takes the fewest
-// rounds of the CUs: four jobs per CU share a key pass and the LDS best
-// (2.97 ms a round of 1024 jobs, 11.3 ms for 4096), a CU with two or one is
-// done sooner (1.78 ms for 512, 1.21 ms for 256; MI355X). So full rounds run
-// at four and what is left at the smallest width that holds it in one round.
-// Eight-wave workgroups of one wave per job, the form before, took 3.5 / 3.7 /
-// 4.2 / 12.0 ms for 256 / 512 / 1024 / 4096 jobs.
-// CMUX keys (one TRGSW per key bit) add the accumulators to the LDS, so two
-// jobs per workgroup are the most; c = 4 and 8 (the default) mix two and one.
+// lvl1 rotation (br_fft_pw.hpp) in the workgroups that fft_split gives.
 template <bool KB, int J, int DPW, int PF, int HELP>
 static void launch_pw_lvl1(const BrJob* jobs, int njobs, uint32_t mu,
                            const FourierKeys<lvl1param>& K, hipStream_t st)
@@ -608,25 +600,15 @@ template <bool KB>
 static void launch_br_lvl1(const BrJob* jobs, int njobs, int c, uint32_t mu,
                            const FourierKeys<lvl1param>& K, hipStream_t st)
 {
-    constexpr int most = KB ? 4 : 2;
-    const int cus = device_cu_count();
-    int full = 0;  // jobs in workgroups of `most`
-    if (c == most && KB) {
-        full = njobs;
-    }
-    else if (c != 1 && c != 2) {
-        full = njobs / (most * cus) * (most * cus);
-        if (njobs - full > most / 2 * cus) full = njobs;
-    }
+    const FftSplit w = fft_split(KB, njobs, c, device_cu_count());
     if constexpr (KB)
-        launch_pw_lvl1<true, 4, 2, 4, 0>(jobs, full, mu, K, st);
+        launch_pw_lvl1<true, 4, 2, 4, 0>(jobs, w.wide, mu, K, st);
     else
-        launch_pw_lvl1<false, 2, 1, 8, 0>(jobs, full, mu, K, st);
-    const int left = njobs - full;
-    if (c == 2 || (c != 1 && left > cus))
-        launch_pw_lvl1<KB, 2, 1, 8, 0>(jobs + full, left, mu, K, st);
+        launch_pw_lvl1<false, 2, 1, 8, 0>(jobs, w.wide, mu, K, st);
+    if (w.width == 2)
+        launch_pw_lvl1<KB, 2, 1, 8, 0>(jobs + w.wide, w.rest, mu, K, st);
     else
-        launch_pw_lvl1<KB, 1, 1, 8, 4>(jobs + full, left, mu, K, st);
+        launch_pw_lvl1<KB, 1, 1, 8, 4>(jobs + w.wide, w.rest, mu, K, st);
 }
 
 // lvl2 rotation. Key bundle (c = 1): br_fft_pw.hpp, one job per workgroup and

@@ -28,4 +28,54 @@ inline int ntt_workgroups(bool cmux, int njobs, int cus)
     return std::min(njobs, rounds * cus);
 }
 
+// Workgroups of an lvl1 FFT batch (br_fft_pw.hpp): its first `wide` jobs in
+// workgroups of `most`, the rest in workgroups of `width`. Key bundle, c = 1, 2, 4:
+// that many jobs per workgroup throughout; else (6, 8, the default) the mix that
+// takes the fewest rounds of the CUs: four jobs per CU share a key pass and the LDS
+// best (2.97 ms a round of 1024 jobs, 11.3 ms for 4096), a CU with two or one is
+// done sooner (1.78 ms for 512, 1.21 ms for 256; MI355X). So full rounds run
+// at four and what is left at the smallest width that holds it in one round.
+// Eight-wave workgroups of one wave per job, the form before, took 3.5 / 3.7 /
+// 4.2 / 12.0 ms for 256 / 512 / 1024 / 4096 jobs.
+// CMUX keys (one TRGSW per key bit) add the accumulators to the LDS, so two
+// jobs per workgroup are the most; c = 4 and 8 (the default) mix two and one.
+struct FftSplit {
+    int most, wide, rest, width;
+    bool operator==(const FftSplit& o) const
+    {
+        return most == o.most && wide == o.wide && rest == o.rest && width == o.width;
+    }
+};
+inline FftSplit fft_split(bool bundle, int njobs, int c, int cus)
+{
+    const int most = bundle ? 4 : 2;
+    int wide = 0;
+    if (c == most) {
+        wide = njobs;
+    }
+    else if (c != 1 && c != 2) {
+        wide = njobs / (most * cus) * (most * cus);
+        if (njobs - wide > most / 2 * cus) wide = njobs;
+    }
+    const int rest = njobs - wide;
+    return FftSplit{most, wide, rest, rest > 0 && (c == 2 || (c != 1 && rest > cus)) ? 2 : 1};
+}
+
+// Times of one launch of a batch over a few repeats.
+struct TunedTime {
+    int c;
+    float best, worst;
+};
+// The c of the fastest of n launches, where the first is the default: another one is
+// taken only if every repeat of it was faster than the default's best, because the
+// pick goes on to smaller batches, where a fixed width can take more than twice the
+// default's time (150 jobs at four a workgroup 2.97 ms, the default 1.21).
+inline int tuned_choice(const TunedTime* t, int n)
+{
+    int pick = 0;
+    for (int i = 1; i < n; i++)
+        if (t[i].worst < t[0].best && t[i].best < t[pick].best) pick = i;
+    return t[pick].c;
+}
+
 }  // namespace cufhe_amd

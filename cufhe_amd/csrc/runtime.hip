@@ -22,6 +22,7 @@
 #include "fft512.hpp"
 #include "ks_gemm.hpp"
 #include "launch.hpp"
+#include "launch_rules.hpp"
 
 namespace cufhe_amd {
 
@@ -897,6 +898,14 @@ int lvl1_pick_c(int c, int nbr)
     if (c == 6) return (k.backend == CUFHE_BACKEND_NTT || k.kb) ? 6 : -1;
     if (c != 1 && c != 2 && c != 4 && c != 8) return -1;
     return c;
+}
+
+// Whether n rotations on the loaded keys are the same launch with c and with d.
+bool lvl1_same_launch(int n, int c, int d)
+{
+    const LevelKeys<lvl1param>& k = state().k1;
+    const int cus = device_cu_count();
+    return k.backend == CUFHE_BACKEND_NTT || fft_split(k.kb, n, c, cus) == fft_split(k.kb, n, d, cus);
 }
 
 size_t lvl1_ks_workspace_bytes(int nks)
@@ -1844,27 +1853,35 @@ int cufhe_autotune_lvl1(int nbootstraps, int* best, float* times_ms, void* strea
     CUFHE_HIP_TRY(hipEventCreate(&mem.e[1]));
     if (times_ms)
         for (int c = 0; c < 9; c++) times_ms[c] = 0.f;
-    int bestc = 0;
-    float bestt = 0.f;
-    for (int c : {1, 2, 4, 6, 8}) {
+    // every launch once among those that are the same at this size; the default first
+    std::vector<TunedTime> timed;
+    for (int c : {8, 1, 2, 4, 6}) {
         if (lvl1_pick_c(c, n) != c) continue;  // not valid for these keys
-        float t = 0.f;
-        for (int rep = 0; rep < 2; rep++) {  // the first launch warms up
+        if (std::none_of(timed.begin(), timed.end(),
+                         [&](const TunedTime& t) { return lvl1_same_launch(n, c, t.c); }))
+            timed.push_back(TunedTime{c, 0.f, 0.f});
+    }
+    for (int rep = 0; rep < 4; rep++) {  // the first one warms up
+        for (TunedTime& w : timed) {
+            float t = 0.f;
             CUFHE_HIP_TRY(hipEventRecord(mem.e[0], st));
-            br_lvl1(d_jobs, n, c, static_cast<uint32_t>(lvl1param::μ), st);
+            br_lvl1(d_jobs, n, w.c, static_cast<uint32_t>(lvl1param::μ), st);
             CUFHE_HIP_TRY(hipEventRecord(mem.e[1], st));
             const int rc = check_launch("autotune rotation");
             if (rc != CUFHE_OK) return rc;
             CUFHE_HIP_TRY(hipEventSynchronize(mem.e[1]));
             CUFHE_HIP_TRY(hipEventElapsedTime(&t, mem.e[0], mem.e[1]));
-        }
-        if (times_ms) times_ms[c] = t;
-        if (bestc == 0 || t < bestt) {
-            bestc = c;
-            bestt = t;
+            if (rep <= 1 || t < w.best) w.best = t;
+            if (rep <= 1 || t > w.worst) w.worst = t;
         }
     }
-    if (bestc == 0) return fail(CUFHE_ERR_STATE, "no rotation kernel for these keys");
+    if (times_ms)
+        for (int c : {1, 2, 4, 6, 8}) {
+            if (lvl1_pick_c(c, n) != c) continue;
+            for (const TunedTime& t : timed)
+                if (lvl1_same_launch(n, c, t.c)) times_ms[c] = t.best;
+        }
+    const int bestc = tuned_choice(timed.data(), static_cast<int>(timed.size()));
     {
         TuneTable& t = tune_table();
         std::lock_guard<std::mutex> g(t.mu);

@@ -211,9 +211,9 @@ int cufhe_plan_jobs_per_group(const cufhe_plan* plan);
  * kernel_ms[0] = key switching, [1] = blind rotation, [2] = combine. */
 int cufhe_plan_run_timed(cufhe_plan* plan, void* stream, float* kernel_ms);
 /* Autotuner of the batched rotation, no reference counterpart: times every
- * rotation kernel / jobs-per-workgroup choice c valid for the loaded lvl1
- * keys (the values of jobs_per_group) on
- * nbootstraps synthetic jobs and records the fastest for that batch size.
+ * jobs_per_group value valid for the loaded lvl1 keys on nbootstraps synthetic
+ * jobs, values that are the same launch at that size once, and records the
+ * fastest: the default (8) unless every repeat of another was faster.
  * Plans, one-shot batches and servers created with jobs_per_group 0 then use
  * the recorded choice of the smallest tuned size >= their batch (else the
  * largest tuned size), and the built-in choice when nothing is tuned; a key

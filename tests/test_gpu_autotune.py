@@ -41,7 +41,7 @@ def test_autotune_picks_a_valid_kernel_and_plans_use_it(keys_lvl1):
     assert np.array_equal(outs[0], outs[1])
     want = [C.TRUTH[o](int(bits[i]), int(bits[n + i])) for i, o in enumerate(names)]
     assert list(C.decrypt_bits(1, keys_lvl1["k1"], outs[0])) == want
-    # a key load clears the record: the built-in choice (8, one wave per job)
+    # a key load clears the record: the built-in choice (8)
     conftest._LOADED_LVL1["tag"] = None
     load_lvl1_keys(("fft", True), keys_lvl1["bk_kb"], keys_lvl1["ksk"],
                    backend=C.BACKEND_FFT, variant=C.BR_KEY_BUNDLE)
@@ -49,3 +49,22 @@ def test_autotune_picks_a_valid_kernel_and_plans_use_it(keys_lvl1):
     plan = C.Plan(gates, d, jobs_per_group=0)
     assert plan.jobs_per_group == 8
     plan.destroy()
+
+
+@pytest.mark.parametrize("bundle", [True, False], ids=["bundle", "cmux"])
+def test_same_launches_tie_and_small_plans_keep_the_mix(keys_lvl1, bundle):
+    """At a whole number of rounds a fixed width is the default's launch: they get one
+    time, the default is recorded, and smaller plans are not held to a fixed width."""
+    C.check(C.lib().cufhe_initialize(), "initialize")
+    conftest._LOADED_LVL1["tag"] = None
+    load_lvl1_keys(("fft", bundle), keys_lvl1["bk_kb" if bundle else "bk"], keys_lvl1["ksk"],
+                   backend=C.BACKEND_FFT, variant=C.BR_KEY_BUNDLE if bundle else C.BR_PLAIN)
+    cus = 256
+    d = C.DeviceBuffer(3 * C.TLWE1_WORDS * 4)
+    for n, same in ((2 * cus, 2), (4 * cus, 4 if bundle else 2), (16 * cus, 4)):
+        best, times = C.autotune_lvl1(n)
+        assert times[8] == times[same] and times.get(6, times[8]) == times[8], (n, times)
+        assert best == 8, (n, times)
+        plan = C.Plan([("NAND", 2, 0, 1, 0)], d)
+        assert plan.jobs_per_group == 8
+        plan.destroy()
