@@ -347,7 +347,7 @@ def workload_kb4096(args):
 
     br_avg_s = statistics.mean(br_ms) / 1e3
     achieved = FLOP_PER_BOOTSTRAP_KB * nbr / br_avg_s / 1e12
-    groups = -(-nbr // best_c)
+    groups = C.lib().cufhe_rotation_workgroups_lvl1(nbr, best_c)
     key_gbps = BK_BYTES_KB * groups / br_avg_s / 1e9
     traffic = measured_traffic("kb4096")
 
@@ -544,9 +544,9 @@ def workload_nttbb(args):
     plain_tput, plain_lat = plain_form(C, gate_fn, [(i,) for i in range(min(args.plain_sample, B))],
                                        args.plain_streams)
     br_avg_s = statistics.mean(br_ms) / 1e3
-    groups = -(-nbr // best_c)
+    groups = C.lib().cufhe_rotation_workgroups_lvl1(nbr, best_c)
     key_gbps = BK_BYTES_NTT_BB * groups / br_avg_s / 1e9
-    valu_g = (NTT_BB_VALU_INSTS_C8 / br_avg_s / 1e9) if best_c == 8 else float("nan")
+    valu_g = (NTT_BB_VALU_INSTS_C8 / br_avg_s / 1e9) if nbr == 4096 else float("nan")
     res = base_result(args, value, total * 1e3 / args.steps, "u32 mod P", {
         "workload": "batched lvl1 NAND/XOR gates, NTT backend (P=2147473409), block-binary "
                     "lvl0 key (blocks of 4), subset key switching, 4096 gates",
@@ -572,7 +572,7 @@ def workload_nttbb(args):
                                              "alpha_bk=2^-24.8, 8 key-noise terms per block (cufhe_amd/noise.py)"},
         "bit_exact_sample": bit_exact,
         # integer-only kernel bound by VALU issue: VALU wave-instructions per
-        # launch (profiles/rotations_trace_and_counters.md, C=8) over
+        # launch (profiles/rotations_trace_and_counters.md) over
         # the live launch time, against one wave-instruction per CU-cycle
         "roofline": {"bound": "valu", "achieved": round(valu_g, 1), "peak": VALU_PEAK_GINST,
                      "unit": "G wave-instr/s", "frac": round(valu_g / VALU_PEAK_GINST, 4),

@@ -104,6 +104,7 @@ def lib():
         "cufhe_memset_d": ([vp, i32, sz, vp], i32),
         "cufhe_memcpy_d2d": ([vp, vp, sz, vp], i32),
         "cufhe_plan_jobs_per_group": ([vp], i32),
+        "cufhe_rotation_workgroups_lvl1": ([i32, i32], i32),
         "cufhe_plan_run_timed": ([vp, vp, ctypes.POINTER(ctypes.c_float)], i32),
         "cufhe_set_key_switch_split": ([i32], i32),
         "cufhe_autotune_lvl1": ([i32, ctypes.POINTER(i32), ctypes.POINTER(ctypes.c_float), vp], i32),

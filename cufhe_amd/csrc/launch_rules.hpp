@@ -45,6 +45,7 @@ struct FftSplit {
     {
         return most == o.most && wide == o.wide && rest == o.rest && width == o.width;
     }
+    int workgroups() const { return (wide + most - 1) / most + (rest + width - 1) / width; }
 };
 inline FftSplit fft_split(bool bundle, int njobs, int c, int cus)
 {

@@ -1895,6 +1895,19 @@ int cufhe_autotune_lvl1(int nbootstraps, int* best, float* times_ms, void* strea
     return CUFHE_OK;
 }
 
+int cufhe_rotation_workgroups_lvl1(int nbootstraps, int jobs_per_group)
+{
+    const LevelKeys<lvl1param>& k = state().k1;
+    if (!k.loaded) return fail(CUFHE_ERR_STATE, "lvl1 keys not loaded");
+    if (nbootstraps < 0) return fail(CUFHE_ERR_ARG, "negative count");
+    if (nbootstraps == 0) return 0;
+    const int c = lvl1_pick_c(jobs_per_group, nbootstraps), cus = device_cu_count();
+    if (c < 0) return fail(CUFHE_ERR_UNSUPPORTED, "unsupported jobs_per_group");
+    if (k.backend == CUFHE_BACKEND_NTT)
+        return ntt_workgroups(k.variant == CUFHE_BR_PLAIN, nbootstraps, cus);
+    return fft_split(k.kb, nbootstraps, c, cus).workgroups();
+}
+
 int cufhe_set_lvl2_jobs_per_group(int c)
 {
     if (c != 1 && c != 2) return fail(CUFHE_ERR_ARG, "lvl2 jobs per workgroup must be 1 or 2");

@@ -221,6 +221,9 @@ int cufhe_plan_run_timed(cufhe_plan* plan, void* stream, float* kernel_ms);
  * times_ms (optional, 9 floats) the rotation ms indexed by c (0 = not
  * valid). Synchronous; allocates scratch for the run. */
 int cufhe_autotune_lvl1(int nbootstraps, int* best, float* times_ms, void* stream);
+/* Workgroups, each of which reads the key once, that nbootstraps lvl1 rotations
+ * with jobs_per_group are launched in on the loaded keys; < 0 on error. */
+int cufhe_rotation_workgroups_lvl1(int nbootstraps, int jobs_per_group);
 /* Tuning knob of the batched (int8 MFMA) key switch, no reference
  * counterpart: the number of waves the digit dimension of each output tile
  * is split over, their partial sums added atomically (1-64); 0 restores the

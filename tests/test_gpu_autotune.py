@@ -68,3 +68,17 @@ def test_same_launches_tie_and_small_plans_keep_the_mix(keys_lvl1, bundle):
         plan = C.Plan([("NAND", 2, 0, 1, 0)], d)
         assert plan.jobs_per_group == 8
         plan.destroy()
+
+
+@pytest.mark.parametrize("bundle, counts", [
+    (True, {(4096, 4): 1024, (4096, 8): 1024, (4096, 0): 1024, (4096, 2): 2048, (150, 8): 150, (1100, 6): 332}),
+    (False, {(4096, 4): 2048, (4096, 1): 4096, (600, 8): 344}),
+], ids=["bundle", "cmux"])
+def test_rotation_workgroups_are_the_launched_ones(keys_lvl1, bundle, counts):
+    C.check(C.lib().cufhe_initialize(), "initialize")
+    conftest._LOADED_LVL1["tag"] = None
+    load_lvl1_keys(("fft", bundle), keys_lvl1["bk_kb" if bundle else "bk"], keys_lvl1["ksk"],
+                   backend=C.BACKEND_FFT, variant=C.BR_KEY_BUNDLE if bundle else C.BR_PLAIN)
+    for (n, c), groups in counts.items():
+        assert C.lib().cufhe_rotation_workgroups_lvl1(n, c) == groups, (n, c)
+    assert C.lib().cufhe_rotation_workgroups_lvl1(10, 3) < 0
