@@ -25,11 +25,6 @@
 
 namespace cufhe_amd {
 
-// Registers of key values kept in flight ahead of the multiply-accumulate.
-#ifndef CUFHE_BR_PREFETCH
-#define CUFHE_BR_PREFETCH 2
-#endif
-
 template <class P>
 inline constexpr size_t kTrgswFourier =
     static_cast<size_t>(TFHEpp::BootstrappingTRGSWRows<P>) * (P::k + 1) * (P::n / 2);
@@ -176,6 +171,7 @@ __device__ __forceinline__ void br_step_fft(AccStore<P>& acc, int j, uint32_t a0
                                             const cplx* partner_spec, const FourierKeys<P>& K)
 {
     static_assert(!(KB && DIRECT), "DIRECT takes a single TRGSW");
+    static_assert(!KB || AccStore<P>::kLds, "key bundle: lvl2");
     constexpr bool kSelf = KB || DIRECT;  // digits of acc itself; result assigned
     using T = typename P::T;
     using S = BrShape<P>;
@@ -234,9 +230,9 @@ __device__ __forceinline__ void br_step_fft(AccStore<P>& acc, int j, uint32_t a0
         struct KeyVals {
             cplx k[2][KB ? 3 : 1];
         };
-        // (Torus64: three registers ahead, measured 3% faster on the lvl02
+        // (key bundle: three registers ahead, measured 3% faster on the lvl02
         // mix than two; four spill)
-        constexpr int PD = KB ? (sizeof(T) == 8 ? 3 : CUFHE_BR_PREFETCH) : R;
+        constexpr int PD = KB ? 3 : R;
         const int q = ps * NB;  // NB == 1: one digit per pass
         auto load_keys = [&](int d) -> KeyVals {
             KeyVals v;

@@ -14,7 +14,7 @@
 //  1. forward: wave (job, component j, qi) turns its DPW digit polynomials
 //     into spectra, each in an LDS buffer that is the transform's scratch too;
 //  2. multiply-accumulate: every wave takes R/W registers' worth of bins
-//     (64 bins each) of its jobs. A key value is loaded from L2 by one wave,
+//     (64 bins each) of all jobs. A key value is loaded from L2 by one wave,
 //     straight into VGPRs, and used for every job: there is no key ring in LDS
 //     and no barrier inside the phase. A lane reads the digit spectra at its
 //     bins and writes the two output spectra over two of them (no other lane
@@ -36,27 +36,22 @@
 
 namespace cufhe_amd {
 
-// J jobs per workgroup; DPW digit polynomials per wave and pass; the L gadget
-// digits go through phases 1-2 in PASSES passes (fewer digit buffers in LDS,
-// the sums stay in VGPRs between them); PF key blocks (three values) are in
-// flight per lane.
-template <class P_, int J_, int PASSES_, int DPW_, int PF_, int HELP_ = 0, bool KB_ = true>
+// J jobs per workgroup; DPW digit polynomials per wave; PF key blocks (three
+// values) are in flight per lane.
+template <class P_, int J_, int DPW_, int PF_, int HELP_ = 0, bool KB_ = true>
 struct PwShape {
     using P = P_;
     using T = typename P::T;
     static constexpr int N = P::n, H = N / 2, R = H / 64, G = R / 8, L = P::l;
     static constexpr bool kLvl1 = sizeof(T) == 4;
-    static constexpr int J = J_, PASSES = PASSES_, DPW = DPW_, PF = PF_;
-    static constexpr int QD = L / PASSES;  // digits per component and pass
-    static constexpr int QW = QD / DPW;    // digit waves per component
+    static constexpr int J = J_, DPW = DPW_, PF = PF_;
+    static constexpr int QW = L / DPW;                // digit waves per component
     static constexpr int WPJ = 2 * QW, FW = J * WPJ;  // transform waves
     static constexpr int HELP = HELP_;                // waves of phase 2 only, and the roots
     static constexpr int W = FW + HELP, NT = 64 * W;
-    static constexpr int SETS = W > R ? W / R : 1;  // wave sets that share the bins
-    static constexpr int JL = J / SETS;             // jobs per wave in phase 2
-    static constexpr int BPL = W > R ? 1 : R / W;   // registers (64-bin groups) per wave
-    static constexpr int BLK = QD * 4;              // key blocks per pass and register
-    static constexpr int NB = BPL * BLK;            // key blocks per pass
+    static constexpr int BPL = R / W;                 // registers (64-bin groups) per wave in phase 2
+    static constexpr int BLK = L * 4;                 // key blocks per register
+    static constexpr int NB = BPL * BLK;              // key blocks
     static constexpr bool KB = KB_;
     static constexpr int NM = KB ? 3 : 1;  // key values of a block: the bundle's members
     static constexpr int STEPS = KB ? lvl0param::n / 2 : lvl0param::n;
@@ -67,23 +62,23 @@ struct PwShape {
     static constexpr int WORDS = kLvl1 ? R : 2 * R;
     static constexpr bool kPrio = J > 1;  // several waves per SIMD meet at the barriers
     // all key blocks of a step in flight before phase 2 (else PF ahead, rolling)
-    static constexpr bool kFull = PASSES == 1 && PF == NB;
+    static constexpr bool kFull = PF == NB;
     // the roots of a job in the idle ends of its digit 1 buffers instead of an array
     static constexpr bool kTail = KB && kLvl1 && QW == 2 && HELP == 0;
     static constexpr bool kBase = KB && !kTail;
     static constexpr int TAB = kLvl1 ? fft512::kTabWords : 3 * 64;
-    static_assert(QW * DPW == QD && QD * PASSES == L && JL * SETS == J, "shape");
-    static_assert(kLvl1 || (DPW == 1 && L == 4 && P::Bgbit == 10), "lvl2 digit words");
-    static_assert(KB || (kLvl1 && PASSES == 1), "CMUX keys: lvl1");
+    static_assert(QW * DPW == L, "shape");
+    static_assert(kLvl1 ? L == 2 && P::Bgbit == 8 : DPW == 1 && L == 4 && P::Bgbit == 10, "digit words");
+    static_assert(KB || kLvl1, "CMUX keys: lvl1");
     static_assert(HELP == 0 || HELP >= 2 * J, "two root waves per job");
     static_assert(!kFull || kLvl1, "the next step's keys are loaded in fft512's hooks");
-    static_assert((W > R ? W % R == 0 : R % W == 0) && NB % PF == 0, "even split");
+    static_assert(BPL * W == R && NB % PF == 0, "even split");
 };
 
 template <class S>
 struct PwShared {
-    cplx buf[S::J * 2 * S::QD][fft_stage::kScratchPad(S::H)];  // [(job * QD + digit) * 2 + j]
-    cplx base[S::kTail ? 1 : S::J][S::NX][S::G][S::kTail ? 1 : 64];                          // E[a (1 - 4 kb)] of a0, a1 (, a0 + a1)
+    cplx buf[S::J * 2 * S::L][fft_stage::kScratchPad(S::H)];  // [(job * L + digit) * 2 + j]
+    cplx base[S::kBase ? S::J : 1][S::NX][S::G][S::kBase ? 64 : 1];  // E[a (1 - 4 kb)] of a0, a1 (, a0 + a1)
     cplx tab[S::TAB];                                          // transform tables
     uint32_t a[S::J][S::NX];
     typename S::T acc[S::KB ? 1 : S::J][2][S::KB ? 1 : S::N];  // CMUX keys: the accumulators
@@ -140,7 +135,7 @@ struct PwWave {
     }
     __device__ __forceinline__ cplx* buf(int s, int comp, int ql) const
     {
-        return sm.buf[(s * S::QD + ql) * 2 + comp];
+        return sm.buf[(s * L + ql) * 2 + comp];
     }
     // Tables behind an offset the compiler cannot see through: their loads
     // stay inside the loop instead of occupying VGPRs across it.
@@ -199,10 +194,10 @@ struct PwWave {
                          {static_cast<uint32_t>(a >> 24), static_cast<uint32_t>(b >> 24)}};
         }
     }
-    // folded digit m of this wave (gadget digit (pass QW + qi) DPW + m) at register r
-    __device__ __forceinline__ cplx digits(int r, int pass, int m) const
+    // folded digit m of this wave (gadget digit qi DPW + m) at register r
+    __device__ __forceinline__ cplx digits(int r, int m) const
     {
-        const int q = (pass * S::QW + qi) * S::DPW + m;
+        const int q = qi * S::DPW + m;
         auto field = [](uint32_t w, int at, int bits) {
             return static_cast<double>(static_cast<int32_t>(__builtin_amdgcn_sbfe(w, at, bits)));
         };
@@ -276,19 +271,19 @@ struct PwWave {
         }
     }
 
-    // Key block b of a pass: register dd, digit, component, output column; its
+    // Key block b of a step: register dd, digit, component, output column; its
     // three bundle members.
     struct KeyBlk {
         cplx k[S::NM];
     };
-    __device__ __forceinline__ KeyBlk load_key(int step, int pass, int b, int d0) const
+    __device__ __forceinline__ KeyBlk load_key(int step, int b, int d0) const
     {
         constexpr size_t TS = kTrgswFourier<P>;
         const int dd = b / S::BLK, ql = (b % S::BLK) / 4, comp = (b / 2) & 1, col = b & 1;
         // wave-uniform address (SGPRs) plus the lane's 32-bit byte offset
         const uint32_t st = __builtin_amdgcn_readfirstlane(step);
         const uint32_t in_step = __builtin_amdgcn_readfirstlane(
-            ((comp * L + pass * S::QD + ql) * 2 + col) * H + (d0 + dd) * 64);
+            ((comp * L + ql) * 2 + col) * H + (d0 + dd) * 64);
         const uint64_t u = reinterpret_cast<uint64_t>(K.bk + st * (S::NM * TS) + in_step);
         using gbytes = const __attribute__((address_space(1))) char*;
         const gbytes p = (gbytes)(
@@ -312,8 +307,7 @@ struct PwWave {
     __device__ __forceinline__ void rotate(bool live, uint32_t bar, T mu, const PwMask& mask)
     {
         constexpr int PF = S::PF, NB = S::NB;
-        const int set = S::W > R ? wave / R : 0;
-        const int d0 = S::W > R ? wave % R : wave * S::BPL;
+        const int d0 = wave * S::BPL;
         const bool fft = live && qi >= 0;
         cplx* const mine = buf(slot, j, (qi < 0 ? 0 : qi) * S::DPW);
         const fft512::Slots slots = fft512::Slots::of(lane);
@@ -354,7 +348,7 @@ struct PwWave {
         const bool early = !S::kFull || qi != 0;
         if (early) {
 #pragma unroll
-            for (int b = 0; b < PF; b++) kv[b] = load_key(0, 0, b, d0);
+            for (int b = 0; b < PF; b++) kv[b] = load_key(0, b, d0);
         }
         __syncthreads();  // the first roots
 #pragma unroll 1
@@ -363,13 +357,13 @@ struct PwWave {
             const int next = it + 1 < S::STEPS ? it + 1 : it;
             // W_8^(a d) of this step: scalar loads, at lvl1 long before their use
             // (at lvl2 the transforms need the SGPRs)
-            cplx w8[S::BPL][S::JL][S::NX];
+            cplx w8[S::BPL][S::J][S::NX];
             auto load_w8 = [&]() {
 #pragma unroll
-                for (int jl = 0; jl < S::JL; jl++)
+                for (int jl = 0; jl < S::J; jl++)
 #pragma unroll
                     for (int m = 0; m < S::NX; m++) {
-                        const uint32_t a = __builtin_amdgcn_readfirstlane(sm.a[set * S::JL + jl][m]);
+                        const uint32_t a = __builtin_amdgcn_readfirstlane(sm.a[jl][m]);
 #pragma unroll
                         for (int dd = 0; dd < S::BPL; dd++) {
                             const int e = (a * static_cast<uint32_t>(d0 + dd)) & 7u;
@@ -385,172 +379,163 @@ struct PwWave {
                 roots = gather(mask.value<P>(na0), mask.value<P>(na1));
                 next_mask(it);
             }
-            cplx s[S::BPL][S::JL][2];
+            cplx s[S::BPL][S::J][2];
 #pragma unroll
             for (int dd = 0; dd < S::BPL; dd++)
 #pragma unroll
-                for (int jl = 0; jl < S::JL; jl++) s[dd][jl][0] = s[dd][jl][1] = cplx{0.0, 0.0};
-#pragma unroll 1
-            for (int pass = 0; pass < S::PASSES; pass++) {
-                const bool last = pass + 1 == S::PASSES;
-                const int after = last ? next : it;
-                const int after_pass = last ? 0 : pass + 1;
-                if constexpr (!S::KB) {
-                    // digits of (X^a - 1) acc
-                    if (fft) {
-                        const uint32_t a = mask.value<P>(na0);
-                        if (more) na0 = mask.load(it + 1);
-                        const T* const src = sm.acc[slot][j];
-#pragma unroll
-                        for (int r = 0; r < R; r++) {
-                            const int i = lane + 64 * r;
-                            // X^a acc at i: acc[(i - a) mod N], negated where bit
-                            // log N of i - a (mod 2N) is set
-                            auto rotated = [&](int k) {
-                                const uint32_t u = static_cast<uint32_t>(k) - a;
-                                const uint32_t neg = 0u - ((u >> P::nbit) & 1u);
-                                return (static_cast<uint32_t>(src[u & (N - 1)]) ^ neg) - neg;
-                            };
-                            const Words v = pack(static_cast<T>(rotated(i)) - src[i],
-                                                 static_cast<T>(rotated(i + H)) - src[i + H]);
-                            words[r] = v.own[0];
-                        }
-                    }
-                }
+                for (int jl = 0; jl < S::J; jl++) s[dd][jl][0] = s[dd][jl][1] = cplx{0.0, 0.0};
+            if constexpr (!S::KB) {
+                // digits of (X^a - 1) acc
                 if (fft) {
-                    if constexpr (S::kLvl1) {
-                        cplx z[S::DPW][8];
-                        cplx* zb[S::DPW];
+                    const uint32_t a = mask.value<P>(na0);
+                    if (more) na0 = mask.load(it + 1);
+                    const T* const src = sm.acc[slot][j];
 #pragma unroll
-                        for (int m = 0; m < S::DPW; m++) {
-                            zb[m] = buf(slot, j, qi * S::DPW + m);
-#pragma unroll
-                            for (int r = 0; r < 8; r++) z[m][r] = digits(r, pass, m);
-                        }
-                        // a third of the key blocks behind each stage's stores: the
-                        // vector memory queue takes 16 cycles a load and CU
-                        fft512::forward<S::DPW, S::kPrio>(z, zb, tables(), slots, lane, [&](int part) {
-                            if constexpr (S::kFull)
-                                if (qi == 0 || S::QW == 1)
-#pragma unroll
-                                    for (int b = 0; b < PF; b++)
-                                        if (b * 3 / PF == part) kv[b] = load_key(it, 0, b, d0);
-                        });
-                    }
-                    else {
-                        using namespace fft_stage;
-                        cplx z[R];
-#pragma unroll
-                        for (int r = 0; r < R; r++) z[r] = digits(r, pass, 0);
-                        const FFTTables tb = lvl2_tables();
-                        wave_prio<true>(3);
-#pragma unroll
-                        for (int r = 1; r < R; r++) z[r] = cmul(z[r], cr(r));
-                        fwd_a_dft<R>(z, tb, lane);
-                        t1_store<R, 2>(z, mine, lane);
-                        wave_lds_sync();
-                        t1_load<R, 2>(z, mine, lane);
-                        wave_lds_sync();
-                        wave_prio<true>(2);
-                        fwd_b<R>(z, tb, lane);
-                        t2_store_cx<R, 2>(z, mine, lane);
-                        wave_lds_sync();
-                        t2_load_xc<R, 2>(z, mine, lane);
-                        wave_lds_sync();
-                        wave_prio<true>(1);
-                        fwd_c<R>(z);
-                        wave_prio<true>(0);
-#pragma unroll
-                        for (int d = 0; d < R; d++) lds_store(&mine[d * 64 + lane], z[d]);
+                    for (int r = 0; r < R; r++) {
+                        const int i = lane + 64 * r;
+                        // X^a acc at i: acc[(i - a) mod N], negated where bit
+                        // log N of i - a (mod 2N) is set
+                        auto rotated = [&](int k) {
+                            const uint32_t u = static_cast<uint32_t>(k) - a;
+                            const uint32_t neg = 0u - ((u >> P::nbit) & 1u);
+                            return (static_cast<uint32_t>(src[u & (N - 1)]) ^ neg) - neg;
+                        };
+                        const Words v = pack(static_cast<T>(rotated(i)) - src[i],
+                                             static_cast<T>(rotated(i + H)) - src[i + H]);
+                        words[r] = v.own[0];
                     }
                 }
-                if constexpr (S::kTail)
-                    if (live && rooter) lds_store(&mine[H + lane], tail_root);
-                if (!fft && S::kFull && !early) {
-                    // no job: the wave still multiplies for the others
+            }
+            if (fft) {
+                if constexpr (S::kLvl1) {
+                    cplx z[S::DPW][8];
+                    cplx* zb[S::DPW];
 #pragma unroll
-                    for (int b = 0; b < PF; b++) kv[b] = load_key(it, 0, b, d0);
+                    for (int m = 0; m < S::DPW; m++) {
+                        zb[m] = buf(slot, j, qi * S::DPW + m);
+#pragma unroll
+                        for (int r = 0; r < 8; r++) z[m][r] = digits(r, m);
+                    }
+                    // a third of the key blocks behind each stage's stores: the
+                    // vector memory queue takes 16 cycles a load and CU
+                    fft512::forward<S::DPW, S::kPrio>(z, zb, tables(), slots, lane, [&](int part) {
+                        if constexpr (S::kFull)
+                            if (qi == 0 || S::QW == 1)
+#pragma unroll
+                                for (int b = 0; b < PF; b++)
+                                    if (b * 3 / PF == part) kv[b] = load_key(it, b, d0);
+                    });
                 }
-                // X^a - 1 at this wave's bins; the roots were published a barrier ago
-                cplx x[S::BPL][S::JL][3];
-                auto make_x = [&]() {
-                    if constexpr (!S::kLvl1) load_w8();
+                else {
+                    using namespace fft_stage;
+                    cplx z[R];
+#pragma unroll
+                    for (int r = 0; r < R; r++) z[r] = digits(r, 0);
+                    const FFTTables tb = lvl2_tables();
+                    wave_prio<true>(3);
+#pragma unroll
+                    for (int r = 1; r < R; r++) z[r] = cmul(z[r], cr(r));
+                    fwd_a_dft<R>(z, tb, lane);
+                    t1_store<R>(z, mine, lane);
+                    wave_lds_sync();
+                    t1_load<R>(z, mine, lane);
+                    wave_lds_sync();
+                    wave_prio<true>(2);
+                    fwd_b<R>(z, tb, lane);
+                    t2_store_cx<R>(z, mine, lane);
+                    wave_lds_sync();
+                    t2_load_xc<R>(z, mine, lane);
+                    wave_lds_sync();
+                    wave_prio<true>(1);
+                    fwd_c<R>(z);
+                    wave_prio<true>(0);
+#pragma unroll
+                    for (int d = 0; d < R; d++) lds_store(&mine[d * 64 + lane], z[d]);
+                }
+            }
+            if constexpr (S::kTail)
+                if (live && rooter) lds_store(&mine[H + lane], tail_root);
+            if (!fft && S::kFull && !early) {
+                // no job: the wave still multiplies for the others
+#pragma unroll
+                for (int b = 0; b < PF; b++) kv[b] = load_key(it, b, d0);
+            }
+            // X^a - 1 at this wave's bins; the roots were published a barrier ago
+            cplx x[S::BPL][S::J][3];
+            auto make_x = [&]() {
+                if constexpr (!S::kLvl1) load_w8();
 #pragma unroll
                 for (int dd = 0; dd < S::BPL; dd++)
 #pragma unroll
-                    for (int jl = 0; jl < S::JL; jl++) {
+                    for (int jl = 0; jl < S::J; jl++) {
                         cplx(&xx)[3] = x[dd][jl];
 #pragma unroll
                         for (int m = 0; m < S::NX; m++)
-                            xx[m] = cmul(lds_load(&root(set * S::JL + jl, m, (d0 + dd) >> 3)[lane]),
-                                         w8[dd][jl][m]);
+                            xx[m] = cmul(lds_load(&root(jl, m, (d0 + dd) >> 3)[lane]), w8[dd][jl][m]);
                         if constexpr (S::NX == 2) xx[2] = cmul(xx[0], xx[1]);
 #pragma unroll
                         for (int m = 0; m < 3; m++) xx[m].x -= 1.0;
                     }
-                };
-                // with helper waves after the barrier: before it, their key
-                // loads were waited for there (one gate 1.35 against 1.25 ms)
-                if constexpr (S::kBase && !S::HELP) make_x();
-                __syncthreads();  // digit spectra are in LDS
-                if constexpr (S::kTail || (S::kBase && S::HELP)) make_x();
-                // the spectra of a (digit, component) are loaded while the one
-                // before it is multiplied
-                constexpr int DN = S::BPL * S::QD * 2;
-                cplx D[2][S::JL];
-                auto load_d = [&](int n, cplx(&dst)[S::JL]) {
-                    const int dd = n / (2 * S::QD), ql = (n / 2) % S::QD, comp = n & 1;
+            };
+            // with helper waves after the barrier: before it, their key
+            // loads were waited for there (one gate 1.35 against 1.25 ms)
+            if constexpr (S::kBase && !S::HELP) make_x();
+            __syncthreads();  // digit spectra are in LDS
+            if constexpr (S::kTail || (S::kBase && S::HELP)) make_x();
+            // the spectra of a (digit, component) are loaded while the one
+            // before it is multiplied
+            constexpr int DN = S::BPL * L * 2;
+            cplx D[2][S::J];
+            auto load_d = [&](int n, cplx(&dst)[S::J]) {
+                const int dd = n / (2 * L), ql = (n / 2) % L, comp = n & 1;
 #pragma unroll
-                    for (int jl = 0; jl < S::JL; jl++)
-                        dst[jl] = lds_load(&buf(set * S::JL + jl, comp, ql)[(d0 + dd) * 64 + lane]);
-                };
-                load_d(0, D[0]);
-                wave_prio<S::kPrio>(3);
+                for (int jl = 0; jl < S::J; jl++)
+                    dst[jl] = lds_load(&buf(jl, comp, ql)[(d0 + dd) * 64 + lane]);
+            };
+            load_d(0, D[0]);
+            wave_prio<S::kPrio>(3);
 #pragma unroll
-                for (int dd = 0; dd < S::BPL; dd++) {
+            for (int dd = 0; dd < S::BPL; dd++) {
 #pragma unroll
-                    for (int ql = 0; ql < S::QD; ql++) {
-                        const double hq = ldexp(1.0, -static_cast<int>((pass * S::QD + ql + 1) * P::Bgbit));
+                for (int ql = 0; ql < L; ql++) {
+                    const double hq = ldexp(1.0, -static_cast<int>((ql + 1) * P::Bgbit));
 #pragma unroll
-                        for (int comp = 0; comp < 2; comp++) {
-                            const int n = (dd * S::QD + ql) * 2 + comp;
-                            if (n + 1 < DN) load_d(n + 1, D[(n + 1) & 1]);
-                            if (n == DN / 4) wave_prio<S::kPrio>(2);
-                            if (n == DN / 2) wave_prio<S::kPrio>(1);
-                            if (n == DN * 3 / 4) wave_prio<S::kPrio>(0);
+                    for (int comp = 0; comp < 2; comp++) {
+                        const int n = (dd * L + ql) * 2 + comp;
+                        if (n + 1 < DN) load_d(n + 1, D[(n + 1) & 1]);
+                        if (n == DN / 4) wave_prio<S::kPrio>(2);
+                        if (n == DN / 2) wave_prio<S::kPrio>(1);
+                        if (n == DN * 3 / 4) wave_prio<S::kPrio>(0);
 #pragma unroll
-                            for (int col = 0; col < 2; col++) {
-                                const int i = dd * S::BLK + ql * 4 + comp * 2 + col;
-                                const KeyBlk cur = kv[i % PF];
-                                if constexpr (!S::kFull)
-                                    kv[i % PF] = i + PF < NB ? load_key(it, pass, i + PF, d0)
-                                                             : load_key(after, after_pass, i + PF - NB, d0);
+                        for (int col = 0; col < 2; col++) {
+                            const int i = dd * S::BLK + ql * 4 + comp * 2 + col;
+                            const KeyBlk cur = kv[i % PF];
+                            if constexpr (!S::kFull)
+                                kv[i % PF] = i + PF < NB ? load_key(it, i + PF, d0) : load_key(next, i + PF - NB, d0);
 #pragma unroll
-                                for (int jl = 0; jl < S::JL; jl++) {
-                                    cplx k = cur.k[0];
-                                    if constexpr (S::KB) {
-                                        k = cplx{comp == col ? hq : 0.0, 0.0};
-                                        cmac(k, cur.k[2], x[dd][jl][1]);
-                                        cmac(k, cur.k[1], x[dd][jl][0]);
-                                        cmac(k, cur.k[0], x[dd][jl][2]);
-                                    }
-                                    cmac(s[dd][jl][col], D[n & 1][jl], k);
+                            for (int jl = 0; jl < S::J; jl++) {
+                                cplx k = cur.k[0];
+                                if constexpr (S::KB) {
+                                    k = cplx{comp == col ? hq : 0.0, 0.0};
+                                    cmac(k, cur.k[2], x[dd][jl][1]);
+                                    cmac(k, cur.k[1], x[dd][jl][0]);
+                                    cmac(k, cur.k[0], x[dd][jl][2]);
                                 }
-                                // the loads of later blocks stay behind this block's products
-                                __builtin_amdgcn_sched_barrier(0);
+                                cmac(s[dd][jl][col], D[n & 1][jl], k);
                             }
+                            // the loads of later blocks stay behind this block's products
+                            __builtin_amdgcn_sched_barrier(0);
                         }
                     }
                 }
-                if (!last) __syncthreads();  // spectra consumed
             }
 #pragma unroll
             for (int dd = 0; dd < S::BPL; dd++)
 #pragma unroll
-                for (int jl = 0; jl < S::JL; jl++)
+                for (int jl = 0; jl < S::J; jl++)
 #pragma unroll
                     for (int col = 0; col < 2; col++)
-                        lds_store(&buf(set * S::JL + jl, col, 0)[(d0 + dd) * 64 + lane], s[dd][jl][col]);
+                        lds_store(&buf(jl, col, 0)[(d0 + dd) * 64 + lane], s[dd][jl][col]);
             __syncthreads();  // output spectra are in the digit 0 buffers
             if (S::KB && S::HELP == 0 && live && rooter && more) {
                 if constexpr (!S::kLvl1) {  // an idle partner wave, short of VGPRs
@@ -563,7 +548,7 @@ struct PwWave {
             // (behind the roots' loads: they return in order)
             if (S::kFull && early) {
 #pragma unroll
-                for (int b = 0; b < PF; b++) kv[b] = load_key(next, 0, b, d0);
+                for (int b = 0; b < PF; b++) kv[b] = load_key(next, b, d0);
             }
             if (live && qi == 0) {
                 cplx z[R];
@@ -577,14 +562,14 @@ struct PwWave {
                     wave_lds_sync();
                     const FFTTables tb = lvl2_tables();
                     inv_a<R>(z);
-                    t2_store_xc<R, 2>(z, mine, lane);
+                    t2_store_xc<R>(z, mine, lane);
                     wave_lds_sync();
-                    t2_load_cx<R, 2>(z, mine, lane);
+                    t2_load_cx<R>(z, mine, lane);
                     wave_lds_sync();
                     inv_b<R>(z, tb, lane);
-                    t1_store_inv<R, 2>(z, mine, lane);
+                    t1_store_inv<R>(z, mine, lane);
                     wave_lds_sync();
-                    t1_load_inv<R, 2>(z, mine, lane);
+                    t1_load_inv<R>(z, mine, lane);
                     wave_lds_sync();
                     inv_c_dft<R>(z, tb, lane);
 #pragma unroll

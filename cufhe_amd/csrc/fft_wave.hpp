@@ -63,16 +63,6 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Hide a uniform pointer's provenance so loads through it are not hoisted
-// out of a loop (keeps loop-invariant twiddle tables out of VGPRs; they
-// are re-read from L1 instead).
-template <class T>
-__device__ __forceinline__ T* opaque_ptr(T* p)
-{
-    asm volatile("" : "+s"(p));
-    return p;
-}
-
 __device__ __forceinline__ cplx lds_load(const cplx* p)
 {
     const double2 v = *reinterpret_cast<const double2*>(p);
@@ -165,25 +155,11 @@ __device__ __forceinline__ void dft_reg(cplx* x)
     for (int i = 0; i < M; i++) x[i] = tmp[i];
 }
 
-// Transpose slots in the wave's scratch (16-byte elements). Rows are 64
-// elements. SWZ: a 16-lane group of a 128-bit LDS access must touch 16
-// distinct 4-bank units; odd rows are swizzled so that the two rows read or
-// written by the same 16 lanes (q = 2m, 2m+1) land in opposite bank halves
-// (conflict-free, at the price of per-lane address registers):
-//   step 1: element (row, col) at row*64 + (col ^ 8*(row&1))
-//   step 2: element (row, c, x) at row*64 + 8*(c ^ (row&1)) + x
-// Without SWZ the same slots without the XOR on the row parity (2-way
-// conflicts between the two rows of a 16-lane group).
-template <bool SWZ>
-__device__ __forceinline__ int fft_t1(int row, int col)
-{
-    return row * 64 + (SWZ ? (col ^ ((row & 1) << 3)) : col);
-}
-template <bool SWZ>
-__device__ __forceinline__ int fft_t2(int row, int c, int x)
-{
-    return row * 64 + ((SWZ ? (c ^ (row & 1)) : c) << 3) + x;
-}
+// Transpose slots of fft_forward / fft_inverse in the wave's scratch of H
+// elements (16 bytes each): step 1 element (row, col), step 2 element (row, c, x).
+// Rows are 64 elements; the two rows of a 16-lane group conflict 2-way.
+__device__ __forceinline__ int fft_t1(int row, int col) { return row * 64 + col; }
+__device__ __forceinline__ int fft_t2(int row, int c, int x) { return row * 64 + (c << 3) + x; }
 
 // Wave issue priority (s_setprio) for transforms run by many waves that
 // meet at workgroup barriers: a transform starts at priority 3 and steps down
@@ -249,34 +225,19 @@ __device__ __forceinline__ TwiddleSeq stage_b_twiddles(const FFTTables& tb, int 
 // transformed it (no expression here can be contracted differently).
 namespace fft_stage {
 
-// Scratch slot layouts of the transposes (16-byte elements). LAY 0 and 1 are
-// fft_t1/fft_t2 without / with the XOR swizzle; LAY 2 pads rows to 72
+// Scratch slots of the transposes (16-byte elements): rows are padded to 72
 // elements and step-2 sub-rows to 9, which is conflict-free for both access
 // patterns of both transposes (a 16-lane group's two rows land 8 elements =
 // half a bank sweep apart) and needs no per-register lane XOR, so one
-// address register serves all eight accesses of a pattern. Scratch for LAY 2
-// is kScratchPad(H) elements.
+// address register serves all eight accesses of a pattern. The scratch is
+// kScratchPad(H) elements.
 constexpr int kPadRow = 72;
 __host__ __device__ constexpr int kScratchPad(int H) { return H / 64 * kPadRow; }
 // step 1: element (row, col)
-template <int LAY>
-__device__ __forceinline__ int slot_t1(int row, int col)
-{
-    if constexpr (LAY == 2)
-        return row * kPadRow + col;
-    else
-        return fft_t1<LAY == 1>(row, col);
-}
+__device__ __forceinline__ int slot_t1(int row, int col) { return row * kPadRow + col; }
 // step 2: element (row, c, x) of the 8 x 8 transpose of lane group `row`:
 // lane x of the group holds register c before, lane c holds register x after
-template <int LAY>
-__device__ __forceinline__ int slot_t2(int row, int c, int x)
-{
-    if constexpr (LAY == 2)
-        return row * kPadRow + c * 9 + x;
-    else
-        return fft_t2<LAY == 1>(row, c, x ^ c);
-}
+__device__ __forceinline__ int slot_t2(int row, int c, int x) { return row * kPadRow + c * 9 + x; }
 
 // (fwd_a behind its products with cr)
 template <int R>
@@ -316,20 +277,20 @@ __device__ __forceinline__ void fwd_a2(cplx (&x)[R], cplx (&y)[R], const FFTTabl
         if (k2 + 1 < R) ts.next();
     }
 }
-template <int R, int LAY>
+template <int R>
 __device__ __forceinline__ void t1_store(const cplx (&x)[R], cplx* lds, int lane)
 {
 #pragma unroll
-    for (int k2 = 0; k2 < R; k2++) lds_store(&lds[slot_t1<LAY>(k2, lane)], x[k2]);
+    for (int k2 = 0; k2 < R; k2++) lds_store(&lds[slot_t1(k2, lane)], x[k2]);
 }
-template <int R, int LAY>
+template <int R>
 __device__ __forceinline__ void t1_load(cplx (&x)[R], const cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
     for (int g = 0; g < R / 8; g++)
 #pragma unroll
-        for (int b = 0; b < 8; b++) x[g * 8 + b] = lds_load(&lds[slot_t1<LAY>(g * 8 + q, 8 * b + lo)]);
+        for (int b = 0; b < 8; b++) x[g * 8 + b] = lds_load(&lds[slot_t1(g * 8 + q, 8 * b + lo)]);
 }
 template <int R>
 __device__ __forceinline__ void fwd_b(cplx (&x)[R], const FFTTables& tb, int lane)
@@ -346,23 +307,23 @@ __device__ __forceinline__ void fwd_b(cplx (&x)[R], const FFTTables& tb, int lan
         }
     }
 }
-template <int R, int LAY>
+template <int R>
 __device__ __forceinline__ void t2_store_cx(const cplx (&x)[R], cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
     for (int g = 0; g < R / 8; g++)
 #pragma unroll
-        for (int c = 0; c < 8; c++) lds_store(&lds[slot_t2<LAY>(g * 8 + q, c, lo)], x[g * 8 + c]);
+        for (int c = 0; c < 8; c++) lds_store(&lds[slot_t2(g * 8 + q, c, lo)], x[g * 8 + c]);
 }
-template <int R, int LAY>
+template <int R>
 __device__ __forceinline__ void t2_load_xc(cplx (&x)[R], const cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
     for (int g = 0; g < R / 8; g++)
 #pragma unroll
-        for (int a = 0; a < 8; a++) x[g * 8 + a] = lds_load(&lds[slot_t2<LAY>(g * 8 + q, lo, a)]);
+        for (int a = 0; a < 8; a++) x[g * 8 + a] = lds_load(&lds[slot_t2(g * 8 + q, lo, a)]);
 }
 template <int R>
 __device__ __forceinline__ void fwd_c(cplx (&x)[R])
@@ -376,23 +337,23 @@ __device__ __forceinline__ void inv_a(cplx (&x)[R])
 #pragma unroll
     for (int g = 0; g < R / 8; g++) dft_reg<8, true>(&x[g * 8]);
 }
-template <int R, int LAY>
+template <int R>
 __device__ __forceinline__ void t2_store_xc(const cplx (&x)[R], cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
     for (int g = 0; g < R / 8; g++)
 #pragma unroll
-        for (int a = 0; a < 8; a++) lds_store(&lds[slot_t2<LAY>(g * 8 + q, lo, a)], x[g * 8 + a]);
+        for (int a = 0; a < 8; a++) lds_store(&lds[slot_t2(g * 8 + q, lo, a)], x[g * 8 + a]);
 }
-template <int R, int LAY>
+template <int R>
 __device__ __forceinline__ void t2_load_cx(cplx (&x)[R], const cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
     for (int g = 0; g < R / 8; g++)
 #pragma unroll
-        for (int c = 0; c < 8; c++) x[g * 8 + c] = lds_load(&lds[slot_t2<LAY>(g * 8 + q, c, lo)]);
+        for (int c = 0; c < 8; c++) x[g * 8 + c] = lds_load(&lds[slot_t2(g * 8 + q, c, lo)]);
 }
 template <int R>
 __device__ __forceinline__ void inv_b(cplx (&x)[R], const FFTTables& tb, int lane)
@@ -410,20 +371,20 @@ __device__ __forceinline__ void inv_b(cplx (&x)[R], const FFTTables& tb, int lan
         dft_reg<8, true>(&x[g * 8]);
     }
 }
-template <int R, int LAY>
+template <int R>
 __device__ __forceinline__ void t1_store_inv(const cplx (&x)[R], cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
     for (int g = 0; g < R / 8; g++)
 #pragma unroll
-        for (int b = 0; b < 8; b++) lds_store(&lds[slot_t1<LAY>(g * 8 + q, 8 * b + lo)], x[g * 8 + b]);
+        for (int b = 0; b < 8; b++) lds_store(&lds[slot_t1(g * 8 + q, 8 * b + lo)], x[g * 8 + b]);
 }
-template <int R, int LAY>
+template <int R>
 __device__ __forceinline__ void t1_load_inv(cplx (&x)[R], const cplx* lds, int lane)
 {
 #pragma unroll
-    for (int k2 = 0; k2 < R; k2++) x[k2] = lds_load(&lds[slot_t1<LAY>(k2, lane)]);
+    for (int k2 = 0; k2 < R; k2++) x[k2] = lds_load(&lds[slot_t1(k2, lane)]);
 }
 // (inv_c before its products with cr)
 template <int R>
@@ -472,13 +433,12 @@ __device__ __forceinline__ void inv_c2(cplx (&x)[R], cplx (&y)[R], const FFTTabl
 // (untwisted). Out: spectrum Z[k] = sum_m (p[m] + i p[m+H]) zeta_k^m with
 // zeta_k = exp(i*pi*(1-4k)/N), in the register layout described above.
 // lds: H complex scratch owned by this wave.
-template <int H, bool SWZ = false, bool PRIO = false>
+template <int H>
 __device__ __forceinline__ void fft_forward(cplx (&x)[H / 64], cplx* lds, const FFTTables& tb)
 {
     constexpr int R = H / 64;
     constexpr int G = R / 8;
     const int lane = threadIdx.x & 63;
-    wave_prio<PRIO>(3);
 #pragma unroll
     for (int r = 1; r < R; r++) x[r] = cmul(x[r], tb.cr[r]);
     dft_reg<R, false>(x);
@@ -491,15 +451,14 @@ __device__ __forceinline__ void fft_forward(cplx (&x)[H / 64], cplx* lds, const 
         }
     }
 #pragma unroll
-    for (int k2 = 0; k2 < R; k2++) lds_store(&lds[fft_t1<SWZ>(k2, lane)], x[k2]);
+    for (int k2 = 0; k2 < R; k2++) lds_store(&lds[fft_t1(k2, lane)], x[k2]);
     wave_lds_sync();
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
     for (int g = 0; g < G; g++)
 #pragma unroll
-        for (int b = 0; b < 8; b++) x[g * 8 + b] = lds_load(&lds[fft_t1<SWZ>(g * 8 + q, 8 * b + lo)]);
+        for (int b = 0; b < 8; b++) x[g * 8 + b] = lds_load(&lds[fft_t1(g * 8 + q, 8 * b + lo)]);
     wave_lds_sync();
-    wave_prio<PRIO>(2);
 #pragma unroll
     for (int g = 0; g < G; g++) {
         dft_reg<8, false>(&x[g * 8]);
@@ -510,43 +469,39 @@ __device__ __forceinline__ void fft_forward(cplx (&x)[H / 64], cplx* lds, const 
             if (c < 7) ts.next();
         }
 #pragma unroll
-        for (int c = 0; c < 8; c++) lds_store(&lds[fft_t2<SWZ>(g * 8 + q, c, lo ^ c)], x[g * 8 + c]);
+        for (int c = 0; c < 8; c++) lds_store(&lds[fft_t2(g * 8 + q, c, lo ^ c)], x[g * 8 + c]);
     }
     wave_lds_sync();
 #pragma unroll
     for (int g = 0; g < G; g++)
 #pragma unroll
-        for (int a = 0; a < 8; a++) x[g * 8 + a] = lds_load(&lds[fft_t2<SWZ>(g * 8 + q, lo, a ^ lo)]);
+        for (int a = 0; a < 8; a++) x[g * 8 + a] = lds_load(&lds[fft_t2(g * 8 + q, lo, a ^ lo)]);
     wave_lds_sync();
-    wave_prio<PRIO>(1);
 #pragma unroll
     for (int g = 0; g < G; g++) dft_reg<8, false>(&x[g * 8]);
-    wave_prio<PRIO>(0);
 }
 
 // Inverse folded transform without the 1/H factor: spectrum in the layout
 // fft_forward produces; result x[r] = H * (p[m] + i p[m+H]), m = lane + 64 r.
-template <int H, bool SWZ = false, bool PRIO = false>
+template <int H>
 __device__ __forceinline__ void fft_inverse(cplx (&x)[H / 64], cplx* lds, const FFTTables& tb)
 {
     constexpr int R = H / 64;
     constexpr int G = R / 8;
     const int lane = threadIdx.x & 63;
     const int lo = lane & 7, q = lane >> 3;
-    wave_prio<PRIO>(3);
 #pragma unroll
     for (int g = 0; g < G; g++) {
         dft_reg<8, true>(&x[g * 8]);
 #pragma unroll
-        for (int a = 0; a < 8; a++) lds_store(&lds[fft_t2<SWZ>(g * 8 + q, lo, a ^ lo)], x[g * 8 + a]);
+        for (int a = 0; a < 8; a++) lds_store(&lds[fft_t2(g * 8 + q, lo, a ^ lo)], x[g * 8 + a]);
     }
     wave_lds_sync();
 #pragma unroll
     for (int g = 0; g < G; g++)
 #pragma unroll
-        for (int c = 0; c < 8; c++) x[g * 8 + c] = lds_load(&lds[fft_t2<SWZ>(g * 8 + q, c, lo ^ c)]);
+        for (int c = 0; c < 8; c++) x[g * 8 + c] = lds_load(&lds[fft_t2(g * 8 + q, c, lo ^ c)]);
     wave_lds_sync();
-    wave_prio<PRIO>(2);
 #pragma unroll
     for (int g = 0; g < G; g++) {
         // undo W_64^(a*c): lane low bits are a here, register index c
@@ -558,13 +513,12 @@ __device__ __forceinline__ void fft_inverse(cplx (&x)[H / 64], cplx* lds, const 
         }
         dft_reg<8, true>(&x[g * 8]);
 #pragma unroll
-        for (int b = 0; b < 8; b++) lds_store(&lds[fft_t1<SWZ>(g * 8 + q, 8 * b + lo)], x[g * 8 + b]);
+        for (int b = 0; b < 8; b++) lds_store(&lds[fft_t1(g * 8 + q, 8 * b + lo)], x[g * 8 + b]);
     }
     wave_lds_sync();
 #pragma unroll
-    for (int k2 = 0; k2 < R; k2++) x[k2] = lds_load(&lds[fft_t1<SWZ>(k2, lane)]);
+    for (int k2 = 0; k2 < R; k2++) x[k2] = lds_load(&lds[fft_t1(k2, lane)]);
     wave_lds_sync();
-    wave_prio<PRIO>(1);
     {
         TwiddleSeq ts = stage_a_twiddles(tb, lane);
 #pragma unroll
@@ -576,79 +530,70 @@ __device__ __forceinline__ void fft_inverse(cplx (&x)[H / 64], cplx* lds, const 
     dft_reg<R, true>(x);
 #pragma unroll
     for (int r = 1; r < R; r++) x[r] = cmulc(x[r], tb.cr[r]);
-    wave_prio<PRIO>(0);
 }
 
 // Two forward transforms by one wave through ONE scratch buffer: the
 // transposes take turns on the scratch while the other transform's register
 // stage runs, so the two dependency chains overlap.
-template <int H, int LAY = 2, bool PRIO = false>
+template <int H>
 __device__ __forceinline__ void fft_forward2(cplx (&x)[H / 64], cplx (&y)[H / 64], cplx* lds,
                                              const FFTTables& tb)
 {
     using namespace fft_stage;
     constexpr int R = H / 64;
     const int lane = threadIdx.x & 63;
-    wave_prio<PRIO>(3);
     fwd_a2<R>(x, y, tb, lane);
-    t1_store<R, LAY>(x, lds, lane);
+    t1_store<R>(x, lds, lane);
     wave_lds_sync();
-    t1_load<R, LAY>(x, lds, lane);
+    t1_load<R>(x, lds, lane);
     wave_lds_sync();
-    t1_store<R, LAY>(y, lds, lane);
+    t1_store<R>(y, lds, lane);
     fwd_b<R>(x, tb, lane);
     wave_lds_sync();
-    t1_load<R, LAY>(y, lds, lane);
+    t1_load<R>(y, lds, lane);
     wave_lds_sync();
-    wave_prio<PRIO>(2);
-    t2_store_cx<R, LAY>(x, lds, lane);
+    t2_store_cx<R>(x, lds, lane);
     fwd_b<R>(y, tb, lane);
     wave_lds_sync();
-    t2_load_xc<R, LAY>(x, lds, lane);
+    t2_load_xc<R>(x, lds, lane);
     wave_lds_sync();
-    wave_prio<PRIO>(1);
-    t2_store_cx<R, LAY>(y, lds, lane);
+    t2_store_cx<R>(y, lds, lane);
     fwd_c<R>(x);
     wave_lds_sync();
-    t2_load_xc<R, LAY>(y, lds, lane);
+    t2_load_xc<R>(y, lds, lane);
     wave_lds_sync();
     fwd_c<R>(y);
-    wave_prio<PRIO>(0);
 }
 
 // Two inverse transforms by one wave through one scratch buffer (as above).
-template <int H, int LAY = 2, bool PRIO = false>
+template <int H>
 __device__ __forceinline__ void fft_inverse2(cplx (&x)[H / 64], cplx (&y)[H / 64], cplx* lds,
                                              const FFTTables& tb)
 {
     using namespace fft_stage;
     constexpr int R = H / 64;
     const int lane = threadIdx.x & 63;
-    wave_prio<PRIO>(3);
     inv_a<R>(x);
-    t2_store_xc<R, LAY>(x, lds, lane);
+    t2_store_xc<R>(x, lds, lane);
     inv_a<R>(y);
     wave_lds_sync();
-    t2_load_cx<R, LAY>(x, lds, lane);
+    t2_load_cx<R>(x, lds, lane);
     wave_lds_sync();
-    t2_store_xc<R, LAY>(y, lds, lane);
+    t2_store_xc<R>(y, lds, lane);
     inv_b<R>(x, tb, lane);
     wave_lds_sync();
-    t2_load_cx<R, LAY>(y, lds, lane);
+    t2_load_cx<R>(y, lds, lane);
     wave_lds_sync();
-    wave_prio<PRIO>(2);
-    t1_store_inv<R, LAY>(x, lds, lane);
+    t1_store_inv<R>(x, lds, lane);
     inv_b<R>(y, tb, lane);
     wave_lds_sync();
-    t1_load_inv<R, LAY>(x, lds, lane);
+    t1_load_inv<R>(x, lds, lane);
     wave_lds_sync();
-    wave_prio<PRIO>(1);
-    t1_store_inv<R, LAY>(y, lds, lane);
+    t1_store_inv<R>(y, lds, lane);
     wave_lds_sync();
-    t1_load_inv<R, LAY>(y, lds, lane);
+    t1_load_inv<R>(y, lds, lane);
     wave_lds_sync();
     inv_c2<R>(x, y, tb, lane);
-    wave_prio<PRIO>(0);
 }
 
 }  // namespace cufhe_amd

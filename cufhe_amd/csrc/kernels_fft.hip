@@ -10,12 +10,6 @@ namespace cufhe_amd {
 
 constexpr int kTlwe0Pad = 640;  // lvl0 TLWE (637 words) padded in LDS
 
-// Occupancy target of the batched blind rotation (waves per SIMD); bounds
-// the VGPR budget the compiler schedules for (3 -> 168 VGPRs).
-#ifndef CUFHE_BR_WAVES_PER_SIMD
-#define CUFHE_BR_WAVES_PER_SIMD 3
-#endif
-
 // ---------------------------------------------------------------------------
 // Polynomial -> Fourier spectra. One wave per polynomial.
 // Reference src/bootstrap_gpu.cu:59-112 (__TRGSW2FFT__): signed torus value
@@ -94,22 +88,23 @@ __global__ __launch_bounds__(256) void k_from_fourier(double* out, const cplx* i
 }
 
 // ---------------------------------------------------------------------------
-// Batched blind rotation: C jobs per workgroup, two waves per job. The
-// workgroups walk the job groups with a grid stride, so a grid that fits on
+// Batched lvl2 rotation with two waves per job (CMUX keys; the key bundle with
+// two jobs per workgroup): C jobs per workgroup. The workgroups walk the job groups with a grid stride, so a grid that fits on
 // the device at once keeps every workgroup on the same rotation step: their
 // key reads then meet in L2 instead of drifting apart as later workgroups
 // start when earlier ones finish.
-template <class P, bool KB, int C>
-__global__ __launch_bounds__(128 * C, (sizeof(typename P::T) == 8 && C > 1) ? 1 : CUFHE_BR_WAVES_PER_SIMD) void k_br_fft(const BrJob* __restrict__ jobs, int njobs,
-                                                     typename P::T mu, FourierKeys<P> K)
+template <bool KB, int C>
+__global__ __launch_bounds__(128 * C, C > 1 ? 1 : 3) void k_br_fft(const BrJob* __restrict__ jobs,
+                                                                   int njobs, uint64_t mu,
+                                                                   FourierKeys<lvl2param> K)
 {
-    using T = typename P::T;
+    using P = lvl2param;
+    using T = uint64_t;
     constexpr int N = P::n, H = N / 2, n0 = lvl0param::n;
-    constexpr bool kL = AccStore<P>::kLds;
     constexpr int NB = BrShape<P>::NB;
     __shared__ cplx sh_spec[2 * C][NB * H];
     __shared__ uint32_t sh_tl0[C][kTlwe0Pad];
-    __shared__ T sh_coef[kL ? 2 * C : 1][kL ? N : 1];
+    __shared__ T sh_coef[2 * C][N];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = wave >> 1, j = wave & 1;
     const int ngroups = (njobs + C - 1) / C;
@@ -127,7 +122,7 @@ __global__ __launch_bounds__(128 * C, (sizeof(typename P::T) == 8 && C > 1) ? 1 
         }
         __syncthreads();
         AccStore<P> acc;
-        if constexpr (kL) acc.lds = sh_coef[wave];
+        acc.lds = sh_coef[wave];
         blind_rotate_fft<P, KB>(sh_tl0[slot], mu, acc, j, sh_spec[wave], sh_spec[wave ^ 1], K);
         if (live) {
             if (jb.flags & kBrOutTrlwe)
@@ -138,16 +133,16 @@ __global__ __launch_bounds__(128 * C, (sizeof(typename P::T) == 8 && C > 1) ? 1 
     }
 }
 
-// Workgroups of k_br_fft<P, KB, C> resident on the device at once (0 if the
+// Workgroups of k_br_fft<KB, C> resident on the device at once (0 if the
 // runtime cannot tell), cached per instance.
-template <class P, bool KB, int C>
+template <bool KB, int C>
 static int br_fft_resident_groups()
 {
     static int cached = -1;
     int v = __atomic_load_n(&cached, __ATOMIC_RELAXED);
     if (v < 0) {
         int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_br_fft<P, KB, C>, 128 * C, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_br_fft<KB, C>, 128 * C, 0) !=
                 hipSuccess ||
             per_cu < 0)
             per_cu = 0;
@@ -188,7 +183,7 @@ __global__ __launch_bounds__(S::NT, WPE) void k_br_fft_pw(const BrJob* __restric
 // The lvl2 shape: eight waves, one digit polynomial each, two 64-bin groups of
 // the products. Four key blocks (12 KiB) in flight a wave: the phase streams
 // 786 KB of key through the CU's L2 path; eight spill.
-using Lvl2Shape = PwShape<lvl2param, 1, 1, 1, 4>;
+using Lvl2Shape = PwShape<lvl2param, 1, 1, 4>;
 
 // ---------------------------------------------------------------------------
 // SampleExtract + key switch lvl1 -> lvl0 of n TRLWEs (reference SEIandKS,
@@ -225,7 +220,7 @@ __global__ __launch_bounds__(512) void k_se_ks_lvl10(uint32_t* out, const uint32
 // single wave and the others only streaming the key; now 1.23 ms (MUX 4.40 ->
 // 1.84 ms).
 template <bool KB, bool MUX>
-using GateShape = PwShape<lvl1param, MUX ? 2 : 1, 1, 1, 8, MUX ? 0 : 4, KB>;
+using GateShape = PwShape<lvl1param, MUX ? 2 : 1, 1, 8, MUX ? 0 : 4, KB>;
 
 // coefficient i of SampleExtractIndex<0> of job `job` (its components lie in
 // the digit 0 buffers after rotate())
@@ -249,7 +244,6 @@ __global__ __launch_bounds__(512, 2) void k_gate_lvl1_pw(
     static_assert(S::NT == 512, "eight waves");
     constexpr int N = P::n, n0 = lvl0param::n;
     constexpr uint32_t mu = static_cast<uint32_t>(P::μ);
-    constexpr uint32_t rnd = kMaskRound<P>;
     __shared__ PwShared<S> sm;
     __shared__ uint32_t sh_tl0[S::J][kTlwe0Pad];
     PwWave<S> w(sm, K, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
@@ -291,10 +285,9 @@ __global__ __launch_bounds__(512, 2) void k_gate_lvl01_pw(
 {
     using P = lvl1param;
     using S = GateShape<KB, MUX>;
-    constexpr int N = P::n, n0 = lvl0param::n;
+    constexpr int N = P::n;
     constexpr uint32_t mu = static_cast<uint32_t>(P::μ);
     constexpr uint32_t mu0 = static_cast<uint32_t>(lvl0param::μ);
-    constexpr uint32_t rnd = kMaskRound<P>;
     __shared__ PwShared<S> sm;
     __shared__ uint32_t sh_res[S::J][N + 4];
     PwWave<S> w(sm, K, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), threadIdx.x & 63);
@@ -591,7 +584,7 @@ template <bool KB, int J, int DPW, int PF, int HELP>
 static void launch_pw_lvl1(const BrJob* jobs, int njobs, uint32_t mu,
                            const FourierKeys<lvl1param>& K, hipStream_t st)
 {
-    using S = PwShape<lvl1param, J, 1, DPW, PF, HELP, KB>;
+    using S = PwShape<lvl1param, J, DPW, PF, HELP, KB>;
     if (njobs > 0)
         hipLaunchKernelGGL((k_br_fft_pw<S, 2>), dim3((njobs + J - 1) / J), dim3(S::NT), 0, st, jobs,
                            njobs, mu, K);
@@ -619,8 +612,8 @@ template <bool KB, int C>
 static void launch_br_two_wave(const BrJob* jobs, int njobs, uint64_t mu,
                                const FourierKeys<lvl2param>& K, hipStream_t st)
 {
-    const int groups = (njobs + C - 1) / C, cap = br_fft_resident_groups<lvl2param, KB, C>();
-    hipLaunchKernelGGL((k_br_fft<lvl2param, KB, C>), dim3(cap > 0 && groups > cap ? cap : groups),
+    const int groups = (njobs + C - 1) / C, cap = br_fft_resident_groups<KB, C>();
+    hipLaunchKernelGGL((k_br_fft<KB, C>), dim3(cap > 0 && groups > cap ? cap : groups),
                        dim3(128 * C), 0, st, jobs, njobs, mu, K);
 }
 template <bool KB>
