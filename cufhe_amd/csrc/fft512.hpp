@@ -42,11 +42,11 @@ struct Root {
 struct Roots {
     Root r1, r2, r3, r3h;
     // for the inverse's scales: r3h.c / r3.c = cos(pi / 4) (1 - t3), and c2 c3
-    __device__ __forceinline__ constexpr double k() const
+    __host__ __device__ __forceinline__ constexpr double k() const
     {
         return 0.70710678118654752440 - 0.70710678118654752440 * r3.t;
     }
-    __device__ __forceinline__ constexpr double c23() const { return r2.c * r3.c; }
+    __host__ __device__ __forceinline__ constexpr double c23() const { return r2.c * r3.c; }
 };
 constexpr int kRootWords = 4;  // 16-byte words of a Roots
 // Table layout, 16-byte words: word w of block b of a level group of B blocks
@@ -55,7 +55,7 @@ constexpr int kTab1 = kRootWords * 8, kTab2 = kRootWords * 64;
 constexpr int kTabWords = kTab1 + kTab2;
 
 template <int B>
-__device__ __forceinline__ Roots load_roots(const cplx* tab, int b)
+__host__ __device__ __forceinline__ Roots load_roots(const cplx* tab, int b)
 {
     const cplx w0 = lds_load(&tab[b]), w1 = lds_load(&tab[B + b]), w2 = lds_load(&tab[2 * B + b]),
                w3 = lds_load(&tab[3 * B + b]);
@@ -63,7 +63,7 @@ __device__ __forceinline__ Roots load_roots(const cplx* tab, int b)
 }
 
 // Roots of levels 1-3: angles pi/4, pi/8, pi/16 and 5 pi/16.
-__device__ __forceinline__ constexpr Roots first_roots()
+__host__ __device__ __forceinline__ constexpr Roots first_roots()
 {
     constexpr double c2 = 0.92387953251128675613, c3 = 0.98078528040323044913,
                      c3h = 0.55557023301960222474;
@@ -75,7 +75,7 @@ __device__ __forceinline__ constexpr Roots first_roots()
 
 // lo = u + s v, hi = u - s v (in place u, v); QUARTER: the root is i s.
 template <bool QUARTER>
-__device__ __forceinline__ void bfly(cplx& u, cplx& v, Root s)
+__host__ __device__ __forceinline__ void bfly(cplx& u, cplx& v, Root s)
 {
     const double p = fma(-s.t, v.y, v.x), q = fma(s.t, v.x, v.y);
     const cplx u0 = u;
@@ -89,7 +89,7 @@ __device__ __forceinline__ void bfly(cplx& u, cplx& v, Root s)
     }
 }
 // Three forward levels on eight registers.
-__device__ __forceinline__ void levels(cplx (&x)[8], const Roots& s)
+__host__ __device__ __forceinline__ void levels(cplx (&x)[8], const Roots& s)
 {
 #pragma unroll
     for (int i = 0; i < 4; i++) bfly<false>(x[i], x[i + 4], s.r1);
@@ -106,7 +106,7 @@ __device__ __forceinline__ void levels(cplx (&x)[8], const Roots& s)
 
 // u = lo + hi, v = conj(s) (lo - hi) / c; QUARTER: the root is i s.
 template <bool QUARTER>
-__device__ __forceinline__ void ibfly(cplx& lo, cplx& hi, double t)
+__host__ __device__ __forceinline__ void ibfly(cplx& lo, cplx& hi, double t)
 {
     const cplx d = csub(lo, hi);
     lo = cadd(lo, hi);
@@ -116,7 +116,7 @@ __device__ __forceinline__ void ibfly(cplx& lo, cplx& hi, double t)
         hi = cplx{fma(-t, d.x, d.y), fma(-t, d.y, -d.x)};
 }
 // The same with hi in units of k times lo's.
-__device__ __forceinline__ void ibfly_scaled(cplx& lo, cplx& hi, double t, double k)
+__host__ __device__ __forceinline__ void ibfly_scaled(cplx& lo, cplx& hi, double t, double k)
 {
     const cplx d = {fma(-k, hi.x, lo.x), fma(-k, hi.y, lo.y)};
     lo = cplx{fma(k, hi.x, lo.x), fma(k, hi.y, lo.y)};
@@ -124,7 +124,7 @@ __device__ __forceinline__ void ibfly_scaled(cplx& lo, cplx& hi, double t, doubl
 }
 // Three inverse levels; register r is left in units of scale(r): the
 // products of c1 (bit 2 of r), c2 (bit 1) and c3 (bit 0).
-__device__ __forceinline__ void ilevels(cplx (&x)[8], const Roots& s)
+__host__ __device__ __forceinline__ void ilevels(cplx (&x)[8], const Roots& s)
 {
     ibfly<false>(x[0], x[1], s.r3.t);
     ibfly<true>(x[2], x[3], s.r3.t);
@@ -140,12 +140,12 @@ __device__ __forceinline__ void ilevels(cplx (&x)[8], const Roots& s)
     ibfly<false>(x[2], x[6], s.r1.t);
     ibfly_scaled(x[3], x[7], s.r1.t, s.k());
 }
-__device__ __forceinline__ constexpr double scale(const Roots& s, int r)
+__host__ __device__ __forceinline__ constexpr double scale(const Roots& s, int r)
 {
     const double low = (r & 3) == 0 ? 1.0 : (r & 3) == 1 ? s.r3.c : (r & 3) == 2 ? s.r2.c : s.c23();
     return r & 4 ? s.r1.c * low : low;
 }
-__device__ __forceinline__ void rescale(cplx (&x)[8], const Roots& s)
+__host__ __device__ __forceinline__ void rescale(cplx (&x)[8], const Roots& s)
 {
 #pragma unroll
     for (int r = 1; r < 8; r++) x[r] = cscale(x[r], scale(s, r));
@@ -156,7 +156,7 @@ __device__ __forceinline__ void rescale(cplx (&x)[8], const Roots& s)
 // register 0 wraps to row 0.
 struct Slots {
     int first, rest;
-    __device__ __forceinline__ static Slots of(int lane)
+    __host__ __device__ __forceinline__ static Slots of(int lane)
     {
         auto rev3 = [](int v) { return ((v & 1) << 2) | (v & 2) | (v >> 2); };
         const int n0 = lane >> 3, n1 = rev3(lane & 7);
@@ -164,7 +164,7 @@ struct Slots {
         const int l = c + 8 * q;
         return Slots{l - (lane == 0 ? 7 * 64 : 0), l + (lane == 0 ? 64 : 0)};
     }
-    __device__ __forceinline__ int at(int a) const
+    __host__ __device__ __forceinline__ int at(int a) const
     {
         const int rev = ((a & 1) << 2) | (a & 2) | (a >> 2);
         return (a == 0 ? first : rest) + (7 - rev) * 64;
@@ -175,14 +175,14 @@ struct Slots {
 // 64, the upper four rows half a bank sweep on; octet o reads row rev3(o).
 // Second, within an octet: 8 x 8 with sub-rows of 9.
 constexpr int kScratch = 576;
-__device__ __forceinline__ constexpr int row1(int r) { return r * 64 + 8 * (r >> 2); }
-__device__ __forceinline__ int octet_row1(int lane)
+__host__ __device__ __forceinline__ constexpr int row1(int r) { return r * 64 + 8 * (r >> 2); }
+__host__ __device__ __forceinline__ int octet_row1(int lane)
 {
     const int o = lane >> 3;
     return row1(((o & 1) << 2) | (o & 2) | (o >> 2)) + (lane & 7);
 }
-__device__ __forceinline__ int sub_a(int lane) { return (lane >> 3) * 72 + (lane & 7); }      // + 9 c
-__device__ __forceinline__ int sub_b(int lane) { return (lane >> 3) * 72 + 9 * (lane & 7); }  // + a
+__host__ __device__ __forceinline__ int sub_a(int lane) { return (lane >> 3) * 72 + (lane & 7); }      // + 9 c
+__host__ __device__ __forceinline__ int sub_b(int lane) { return (lane >> 3) * 72 + 9 * (lane & 7); }  // + a
 
 // Forward transforms of M polynomials held by one wave (x[p][r]: folded value
 // lane + 64 r), each through a buffer of its own that receives its spectrum in

@@ -23,6 +23,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 #include <type_traits>
 #include <utility>
@@ -33,25 +34,25 @@ struct cplx {
     double x, y;
 };
 
-__device__ __forceinline__ cplx cadd(cplx a, cplx b) { return {a.x + b.x, a.y + b.y}; }
-__device__ __forceinline__ cplx csub(cplx a, cplx b) { return {a.x - b.x, a.y - b.y}; }
-__device__ __forceinline__ cplx cmul(cplx a, cplx b)
+__host__ __device__ __forceinline__ cplx cadd(cplx a, cplx b) { return {a.x + b.x, a.y + b.y}; }
+__host__ __device__ __forceinline__ cplx csub(cplx a, cplx b) { return {a.x - b.x, a.y - b.y}; }
+__host__ __device__ __forceinline__ cplx cmul(cplx a, cplx b)
 {
     return {fma(a.x, b.x, -a.y * b.y), fma(a.x, b.y, a.y * b.x)};
 }
-__device__ __forceinline__ cplx cmulc(cplx a, cplx b)  // a * conj(b)
+__host__ __device__ __forceinline__ cplx cmulc(cplx a, cplx b)  // a * conj(b)
 {
     return {fma(a.x, b.x, a.y * b.y), fma(a.y, b.x, -a.x * b.y)};
 }
 // acc += a * b
-__device__ __forceinline__ void cmac(cplx& acc, cplx a, cplx b)
+__host__ __device__ __forceinline__ void cmac(cplx& acc, cplx a, cplx b)
 {
     acc.x = fma(a.x, b.x, acc.x);
     acc.x = fma(-a.y, b.y, acc.x);
     acc.y = fma(a.x, b.y, acc.y);
     acc.y = fma(a.y, b.x, acc.y);
 }
-__device__ __forceinline__ cplx cscale(cplx a, double s) { return {a.x * s, a.y * s}; }
+__host__ __device__ __forceinline__ cplx cscale(cplx a, double s) { return {a.x * s, a.y * s}; }
 
 // Order LDS traffic of one wavefront: every lane's earlier LDS accesses are
 // complete and visible before any later one (LDS ops of a wave execute in
@@ -63,24 +64,24 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ cplx lds_load(const cplx* p)
+__host__ __device__ __forceinline__ cplx lds_load(const cplx* p)
 {
     const double2 v = *reinterpret_cast<const double2*>(p);
     return {v.x, v.y};
 }
-__device__ __forceinline__ void lds_store(cplx* p, cplx v)
+__host__ __device__ __forceinline__ void lds_store(cplx* p, cplx v)
 {
     *reinterpret_cast<double2*>(p) = make_double2(v.x, v.y);
 }
 
 // Compile-time loop: f(std::integral_constant<int, I>{}) for I in [0, N).
 template <typename F, int... Is>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, Is...>)
+__host__ __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, Is...>)
 {
     (f(std::integral_constant<int, Is>{}), ...);
 }
 template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f)
+__host__ __device__ __forceinline__ void static_for(F&& f)
 {
     static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
@@ -99,7 +100,7 @@ __host__ __device__ constexpr double sin16(int e) { return cos16(e + 12); }
 // Multiply by W_M^e = exp(-2*pi*i*e/M) (INV: exp(+2*pi*i*e/M)), e constant,
 // M in {2, 4, 8, 16}. Multiples of a quarter turn are exact swaps.
 template <int M, int E, bool INV>
-__device__ __forceinline__ cplx twiddle_const(cplx v)
+__host__ __device__ __forceinline__ cplx twiddle_const(cplx v)
 {
     constexpr int e16 = (E * (16 / M)) & 15;
     if constexpr (e16 == 0) {
@@ -124,7 +125,7 @@ __device__ __forceinline__ cplx twiddle_const(cplx v)
 
 // In-register M-point DFT (radix-2 DIF, natural order in and out).
 template <int M, bool INV>
-__device__ __forceinline__ void dft_reg(cplx* x)
+__host__ __device__ __forceinline__ void dft_reg(cplx* x)
 {
     static_for<4>([&](auto sc) {
         constexpr int half = (M >> 1) >> decltype(sc)::value;
@@ -158,8 +159,8 @@ __device__ __forceinline__ void dft_reg(cplx* x)
 // Transpose slots of fft_forward / fft_inverse in the wave's scratch of H
 // elements (16 bytes each): step 1 element (row, col), step 2 element (row, c, x).
 // Rows are 64 elements; the two rows of a 16-lane group conflict 2-way.
-__device__ __forceinline__ int fft_t1(int row, int col) { return row * 64 + col; }
-__device__ __forceinline__ int fft_t2(int row, int c, int x) { return row * 64 + (c << 3) + x; }
+__host__ __device__ __forceinline__ int fft_t1(int row, int col) { return row * 64 + col; }
+__host__ __device__ __forceinline__ int fft_t2(int row, int c, int x) { return row * 64 + (c << 3) + x; }
 
 // Wave issue priority (s_setprio) for transforms run by many waves that
 // meet at workgroup barriers: a transform starts at priority 3 and steps down
@@ -207,13 +208,13 @@ struct FFTTables {
 //   stage B: tw64[c*8 + a]  = tw64[8 + a]^c        (c = 1 .. 7)
 struct TwiddleSeq {
     cplx t, w;
-    __device__ __forceinline__ void next() { t = cmul(t, w); }
+    __host__ __device__ __forceinline__ void next() { t = cmul(t, w); }
 };
-__device__ __forceinline__ TwiddleSeq stage_a_twiddles(const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ TwiddleSeq stage_a_twiddles(const FFTTables& tb, int lane)
 {
     return TwiddleSeq{tb.twl[lane], tb.tws[lane]};
 }
-__device__ __forceinline__ TwiddleSeq stage_b_twiddles(const FFTTables& tb, int lo)
+__host__ __device__ __forceinline__ TwiddleSeq stage_b_twiddles(const FFTTables& tb, int lo)
 {
     const cplx w = tb.tw64[8 + lo];
     return TwiddleSeq{w, w};
@@ -222,7 +223,8 @@ __device__ __forceinline__ TwiddleSeq stage_b_twiddles(const FFTTables& tb, int 
 // Stages of the transforms for the paired forms (fft_forward2 /
 // fft_inverse2): the operations of fft_forward / fft_inverse split at the
 // transposes, so a polynomial's spectrum is bit-identical whichever form
-// transformed it (no expression here can be contracted differently).
+// transformed it (no expression here can be contracted differently). They run
+// on the host too, a lane at a time, for the tests of their rounding.
 namespace fft_stage {
 
 // Scratch slots of the transposes (16-byte elements): rows are padded to 72
@@ -234,14 +236,14 @@ namespace fft_stage {
 constexpr int kPadRow = 72;
 __host__ __device__ constexpr int kScratchPad(int H) { return H / 64 * kPadRow; }
 // step 1: element (row, col)
-__device__ __forceinline__ int slot_t1(int row, int col) { return row * kPadRow + col; }
+__host__ __device__ __forceinline__ int slot_t1(int row, int col) { return row * kPadRow + col; }
 // step 2: element (row, c, x) of the 8 x 8 transpose of lane group `row`:
 // lane x of the group holds register c before, lane c holds register x after
-__device__ __forceinline__ int slot_t2(int row, int c, int x) { return row * kPadRow + c * 9 + x; }
+__host__ __device__ __forceinline__ int slot_t2(int row, int c, int x) { return row * kPadRow + c * 9 + x; }
 
 // (fwd_a behind its products with cr)
 template <int R>
-__device__ __forceinline__ void fwd_a_dft(cplx (&x)[R], const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ void fwd_a_dft(cplx (&x)[R], const FFTTables& tb, int lane)
 {
     dft_reg<R, false>(x);
     TwiddleSeq ts = stage_a_twiddles(tb, lane);
@@ -252,7 +254,7 @@ __device__ __forceinline__ void fwd_a_dft(cplx (&x)[R], const FFTTables& tb, int
     }
 }
 template <int R>
-__device__ __forceinline__ void fwd_a(cplx (&x)[R], const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ void fwd_a(cplx (&x)[R], const FFTTables& tb, int lane)
 {
 #pragma unroll
     for (int r = 1; r < R; r++) x[r] = cmul(x[r], tb.cr[r]);
@@ -260,7 +262,7 @@ __device__ __forceinline__ void fwd_a(cplx (&x)[R], const FFTTables& tb, int lan
 }
 // fwd_a of two transforms with each twiddle read once
 template <int R>
-__device__ __forceinline__ void fwd_a2(cplx (&x)[R], cplx (&y)[R], const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ void fwd_a2(cplx (&x)[R], cplx (&y)[R], const FFTTables& tb, int lane)
 {
 #pragma unroll
     for (int r = 1; r < R; r++) {
@@ -278,13 +280,13 @@ __device__ __forceinline__ void fwd_a2(cplx (&x)[R], cplx (&y)[R], const FFTTabl
     }
 }
 template <int R>
-__device__ __forceinline__ void t1_store(const cplx (&x)[R], cplx* lds, int lane)
+__host__ __device__ __forceinline__ void t1_store(const cplx (&x)[R], cplx* lds, int lane)
 {
 #pragma unroll
     for (int k2 = 0; k2 < R; k2++) lds_store(&lds[slot_t1(k2, lane)], x[k2]);
 }
 template <int R>
-__device__ __forceinline__ void t1_load(cplx (&x)[R], const cplx* lds, int lane)
+__host__ __device__ __forceinline__ void t1_load(cplx (&x)[R], const cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
@@ -293,7 +295,7 @@ __device__ __forceinline__ void t1_load(cplx (&x)[R], const cplx* lds, int lane)
         for (int b = 0; b < 8; b++) x[g * 8 + b] = lds_load(&lds[slot_t1(g * 8 + q, 8 * b + lo)]);
 }
 template <int R>
-__device__ __forceinline__ void fwd_b(cplx (&x)[R], const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ void fwd_b(cplx (&x)[R], const FFTTables& tb, int lane)
 {
     const int lo = lane & 7;
 #pragma unroll
@@ -308,7 +310,7 @@ __device__ __forceinline__ void fwd_b(cplx (&x)[R], const FFTTables& tb, int lan
     }
 }
 template <int R>
-__device__ __forceinline__ void t2_store_cx(const cplx (&x)[R], cplx* lds, int lane)
+__host__ __device__ __forceinline__ void t2_store_cx(const cplx (&x)[R], cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
@@ -317,7 +319,7 @@ __device__ __forceinline__ void t2_store_cx(const cplx (&x)[R], cplx* lds, int l
         for (int c = 0; c < 8; c++) lds_store(&lds[slot_t2(g * 8 + q, c, lo)], x[g * 8 + c]);
 }
 template <int R>
-__device__ __forceinline__ void t2_load_xc(cplx (&x)[R], const cplx* lds, int lane)
+__host__ __device__ __forceinline__ void t2_load_xc(cplx (&x)[R], const cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
@@ -326,19 +328,19 @@ __device__ __forceinline__ void t2_load_xc(cplx (&x)[R], const cplx* lds, int la
         for (int a = 0; a < 8; a++) x[g * 8 + a] = lds_load(&lds[slot_t2(g * 8 + q, lo, a)]);
 }
 template <int R>
-__device__ __forceinline__ void fwd_c(cplx (&x)[R])
+__host__ __device__ __forceinline__ void fwd_c(cplx (&x)[R])
 {
 #pragma unroll
     for (int g = 0; g < R / 8; g++) dft_reg<8, false>(&x[g * 8]);
 }
 template <int R>
-__device__ __forceinline__ void inv_a(cplx (&x)[R])
+__host__ __device__ __forceinline__ void inv_a(cplx (&x)[R])
 {
 #pragma unroll
     for (int g = 0; g < R / 8; g++) dft_reg<8, true>(&x[g * 8]);
 }
 template <int R>
-__device__ __forceinline__ void t2_store_xc(const cplx (&x)[R], cplx* lds, int lane)
+__host__ __device__ __forceinline__ void t2_store_xc(const cplx (&x)[R], cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
@@ -347,7 +349,7 @@ __device__ __forceinline__ void t2_store_xc(const cplx (&x)[R], cplx* lds, int l
         for (int a = 0; a < 8; a++) lds_store(&lds[slot_t2(g * 8 + q, lo, a)], x[g * 8 + a]);
 }
 template <int R>
-__device__ __forceinline__ void t2_load_cx(cplx (&x)[R], const cplx* lds, int lane)
+__host__ __device__ __forceinline__ void t2_load_cx(cplx (&x)[R], const cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
@@ -356,7 +358,7 @@ __device__ __forceinline__ void t2_load_cx(cplx (&x)[R], const cplx* lds, int la
         for (int c = 0; c < 8; c++) x[g * 8 + c] = lds_load(&lds[slot_t2(g * 8 + q, c, lo)]);
 }
 template <int R>
-__device__ __forceinline__ void inv_b(cplx (&x)[R], const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ void inv_b(cplx (&x)[R], const FFTTables& tb, int lane)
 {
     const int lo = lane & 7;
 #pragma unroll
@@ -372,7 +374,7 @@ __device__ __forceinline__ void inv_b(cplx (&x)[R], const FFTTables& tb, int lan
     }
 }
 template <int R>
-__device__ __forceinline__ void t1_store_inv(const cplx (&x)[R], cplx* lds, int lane)
+__host__ __device__ __forceinline__ void t1_store_inv(const cplx (&x)[R], cplx* lds, int lane)
 {
     const int lo = lane & 7, q = lane >> 3;
 #pragma unroll
@@ -381,14 +383,14 @@ __device__ __forceinline__ void t1_store_inv(const cplx (&x)[R], cplx* lds, int 
         for (int b = 0; b < 8; b++) lds_store(&lds[slot_t1(g * 8 + q, 8 * b + lo)], x[g * 8 + b]);
 }
 template <int R>
-__device__ __forceinline__ void t1_load_inv(cplx (&x)[R], const cplx* lds, int lane)
+__host__ __device__ __forceinline__ void t1_load_inv(cplx (&x)[R], const cplx* lds, int lane)
 {
 #pragma unroll
     for (int k2 = 0; k2 < R; k2++) x[k2] = lds_load(&lds[slot_t1(k2, lane)]);
 }
 // (inv_c before its products with cr)
 template <int R>
-__device__ __forceinline__ void inv_c_dft(cplx (&x)[R], const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ void inv_c_dft(cplx (&x)[R], const FFTTables& tb, int lane)
 {
     {
         TwiddleSeq ts = stage_a_twiddles(tb, lane);
@@ -401,7 +403,7 @@ __device__ __forceinline__ void inv_c_dft(cplx (&x)[R], const FFTTables& tb, int
     dft_reg<R, true>(x);
 }
 template <int R>
-__device__ __forceinline__ void inv_c(cplx (&x)[R], const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ void inv_c(cplx (&x)[R], const FFTTables& tb, int lane)
 {
     inv_c_dft<R>(x, tb, lane);
 #pragma unroll
@@ -409,7 +411,7 @@ __device__ __forceinline__ void inv_c(cplx (&x)[R], const FFTTables& tb, int lan
 }
 // inv_c of two transforms with each twiddle read once
 template <int R>
-__device__ __forceinline__ void inv_c2(cplx (&x)[R], cplx (&y)[R], const FFTTables& tb, int lane)
+__host__ __device__ __forceinline__ void inv_c2(cplx (&x)[R], cplx (&y)[R], const FFTTables& tb, int lane)
 {
     TwiddleSeq ts = stage_a_twiddles(tb, lane);
 #pragma unroll

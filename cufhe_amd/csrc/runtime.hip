@@ -19,7 +19,7 @@
 #include "br_ntt.hpp"
 #include "br_ntt64.hpp"
 #include "engine.hpp"
-#include "fft512.hpp"
+#include "fft_tables.hpp"
 #include "ks_gemm.hpp"
 #include "launch.hpp"
 #include "launch_rules.hpp"
@@ -109,80 +109,21 @@ State& state()
     return s;
 }
 
-// exp(i*pi*t/N) for t in [0, 2N), computed in long double.
-std::vector<cplx> e2n_table(int N)
-{
-    std::vector<cplx> e(2 * N);
-    const long double pi = 3.141592653589793238462643383279502884L;
-    for (int t = 0; t < 2 * N; t++) {
-        const long double a = pi * static_cast<long double>(t) / static_cast<long double>(N);
-        e[t] = cplx{static_cast<double>(cosl(a)), static_cast<double>(sinl(a))};
-    }
-    // exact values on the axes
-    e[0] = {1.0, 0.0};
-    e[N / 2] = {0.0, 1.0};
-    e[N] = {-1.0, 0.0};
-    e[3 * N / 2] = {0.0, -1.0};
-    // Store each root as the FP64 product of e[64 (t >> 6)] and e[t & 63],
-    // rounded exactly as the device's cmul rounds it: kernels that rebuild
-    // e[t] from those two short tables (in LDS) and kernels that gather e[t]
-    // then see identical values. Entries t < 64 and t = 64u are unchanged.
-    std::vector<cplx> p(2 * N);
-    for (int t = 0; t < 2 * N; t++) {
-        const cplx a = e[64 * (t >> 6)], b = e[t & 63];
-        p[t] = cplx{std::fma(a.x, b.x, -a.y * b.y), std::fma(a.x, b.y, a.y * b.x)};
-    }
-    return p;
-}
-
-// fft512.hpp's root tables: per block of angle theta (the roots of X^n -
-// exp(i theta)) cos and tan of theta / 2, / 4, / 8 and / 8 + pi / 4.
-std::vector<cplx> fft512_tables()
-{
-    std::vector<cplx> t(fft512::kTabWords);
-    auto fill = [&](cplx* out, int blocks, auto n_of) {
-        for (int b = 0; b < blocks; b++) {
-            // theta = pi / (2 blocks) * (1 + 4 n): 8 blocks after three levels, 64 after six
-            const long double pi = 3.14159265358979323846264338327950288L;
-            const long double theta = pi * (1 + 4 * n_of(b)) / (2 * blocks);
-            const long double ang[4] = {theta / 2, theta / 4, theta / 8, theta / 8 + pi / 4};
-            for (int w = 0; w < 4; w++)
-                out[w * blocks + b] = cplx{static_cast<double>(cosl(ang[w])), static_cast<double>(tanl(ang[w]))};
-        }
-    };
-    auto rev3 = [](int v) { return ((v & 1) << 2) | (v & 2) | (v >> 2); };
-    fill(t.data(), 8, [&](int o) { return o; });
-    fill(t.data() + fft512::kTab1, 64, [&](int l) { return (l >> 3) + 8 * rev3(l & 7); });
-    return t;
-}
-
 template <class P>
 int build_tables(TableSet<P>& ts)
 {
-    constexpr int N = P::n, H = N / 2, R = H / 64;
-    const std::vector<cplx> E = e2n_table(N);
-    auto at = [&](long long t) { return E[static_cast<size_t>(((t % (2 * N)) + 2 * N) % (2 * N))]; };
-    std::vector<cplx> twl(R * 64), tw64(64), cr(R), tws(64);
-    // twl[k2*64+l] = exp(i*pi*l/N) * exp(-2*pi*i*l*k2/H) = E[l*(1 - 4*k2)]
-    for (int k2 = 0; k2 < R; k2++)
-        for (int l = 0; l < 64; l++) twl[k2 * 64 + l] = at(static_cast<long long>(l) * (1 - 4 * k2));
-    // tw64[c*8+a] = exp(-2*pi*i*a*c/64) = E[-(2N/64)*a*c]
-    for (int c = 0; c < 8; c++)
-        for (int a = 0; a < 8; a++) tw64[c * 8 + a] = at(-static_cast<long long>(2 * N / 64) * a * c);
-    // tws[l] = exp(-2*pi*i*l/H) = E[-4 l]
-    for (int l = 0; l < 64; l++) tws[l] = at(-4LL * l);
-    // cr[r] = exp(i*pi*64*r/N) = E[64 r]
-    for (int r = 0; r < R; r++) cr[r] = at(64LL * r);
+    constexpr int N = P::n;
+    const FoldedTables t(N);
     auto up = [](cplx** dst, const std::vector<cplx>& v) -> hipError_t {
         hipError_t e = hipMalloc(reinterpret_cast<void**>(dst), v.size() * sizeof(cplx));
         if (e != hipSuccess) return e;
         return hipMemcpy(*dst, v.data(), v.size() * sizeof(cplx), hipMemcpyHostToDevice);
     };
-    CUFHE_HIP_TRY(up(&ts.twl, twl));
-    CUFHE_HIP_TRY(up(&ts.tw64, tw64));
-    CUFHE_HIP_TRY(up(&ts.cr, cr));
-    CUFHE_HIP_TRY(up(&ts.tws, tws));
-    CUFHE_HIP_TRY(up(&ts.e2n, E));
+    CUFHE_HIP_TRY(up(&ts.twl, t.twl));
+    CUFHE_HIP_TRY(up(&ts.tw64, t.tw64));
+    CUFHE_HIP_TRY(up(&ts.cr, t.cr));
+    CUFHE_HIP_TRY(up(&ts.tws, t.tws));
+    CUFHE_HIP_TRY(up(&ts.e2n, t.e2n));
     if constexpr (N == 1024) CUFHE_HIP_TRY(up(&ts.roots, fft512_tables()));
     return CUFHE_OK;
 }

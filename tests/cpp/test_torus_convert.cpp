@@ -1,6 +1,7 @@
-// double_to_torus on the host: rint(v) mod 2^w of doubles around every place where
-// its steps change (ties, the 2^31 / 2^32 / 2^63 / 2^64 edges, large values),
-// against integer arithmetic on the double's mantissa. Runs without a GPU.
+// double_to_torus and turns_to_torus32 on the host: rint(v) mod 2^w of doubles
+// around every place where their steps change (ties, the 2^31 / 2^32 / 2^63 / 2^64
+// edges, half turns, large values), against integer arithmetic on the double's
+// mantissa. Runs without a GPU.
 #include "../../cufhe_amd/csrc/device_common.hpp"
 
 #include <cmath>
@@ -38,6 +39,12 @@ static void check(double v)
         std::exit(1);
     }
     checked++;
+    // the same value given in turns (2^-32 is a power of two: no rounding)
+    const uint32_t turns = cufhe_amd::turns_to_torus32(v * 0x1p-32);
+    if (turns != static_cast<uint32_t>(want)) {
+        std::printf("turns %a: %08x, not %08x\n", v * 0x1p-32, turns, static_cast<uint32_t>(want));
+        std::exit(1);
+    }
     if (std::fabs(v) >= 2251799813685248.0) return;  // 2^51: the lvl1 products stay below
     const uint32_t got32 = cufhe_amd::double_to_torus<uint32_t>(v);
     if (got32 != static_cast<uint32_t>(want)) {
