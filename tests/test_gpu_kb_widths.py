@@ -10,10 +10,12 @@ from conftest import load_lvl1_keys
 
 pytestmark = pytest.mark.gpu
 
+MOST = 1537
+
 
 @pytest.fixture(scope="module", params=[True, False], ids=["bundle", "cmux"])
 def rotations(request, keys_lvl1):
-    """1027 random lvl0 samples, some with masks that round to 0, N and 2N - 1,
+    """MOST random lvl0 samples, some with masks that round to 0, N and 2N - 1,
     and their rotations by the one-job workgroups."""
     kb = request.param
     C.check(C.lib().cufhe_initialize(), "initialize")
@@ -21,7 +23,7 @@ def rotations(request, keys_lvl1):
     load_lvl1_keys(("fft", kb), bk, keys_lvl1["ksk"], backend=C.BACKEND_FFT,
                    variant=C.BR_KEY_BUNDLE if kb else C.BR_PLAIN)
     rng = np.random.default_rng(61)
-    tl0 = rng.integers(0, 2**32, (1027, 637), dtype=np.uint64).astype(np.uint32)
+    tl0 = rng.integers(0, 2**32, (MOST, 637), dtype=np.uint64).astype(np.uint32)
     tl0[0] = 0
     tl0[1] = np.uint32(1 << 31)
     tl0[2] = np.uint32(0xFFFFFFFF)
@@ -38,13 +40,14 @@ def _run(tl0, c):
 def test_one_job_workgroups_equal_the_exact_oracle(rotations):
     # integers: the FP64 product is within a small fraction of a unit of them
     kb, bk, tl0, out = rotations
-    for i in (0, 1, 2, 3, 1026):
+    for i in (0, 1, 2, 3, 1026, MOST - 1):
         acc = O.blind_rotate(1, O.EXACT, kb, tl0[i], bk, C.MU1)
         assert np.array_equal(out[i], O.sample_extract(1, acc)), i
 
 
 @pytest.mark.parametrize("c", [0, 2, 4])
-@pytest.mark.parametrize("n", [1, 2, 3, 5, 255, 256, 257, 512, 513, 1024, 1027])
+# 1281 to 1536: with the key bundle, two jobs per workgroup behind full rounds of four
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 255, 256, 257, 512, 513, 1024, 1027, 1281, 1300, 1536, MOST])
 def test_widths_agree(rotations, c, n):
     _, _, tl0, out = rotations
     assert np.array_equal(_run(tl0[:n], c), out[:n])
