@@ -29,9 +29,9 @@
 // shortens a short batch's step.
 //
 // Measured against two waves per job and two jobs per workgroup (rotations of
-// 1 / 1000 / 4096 jobs, ms): block-binary 2.90 / 4.37 / 14.0 -> 1.30 / 2.5 / 8.35,
-// key bundle 5.3 / 7.7 / 25.7 -> 2.8 / 5.1 / 17.6, plain 9.2 / 12.3 / 38.2 ->
-// 5.3 / 8.4 / 29.4 (the last two before the issue priorities).
+// 1 / 1024 / 4096 jobs, ms): block-binary 2.92 / 4.28 / 14.1 -> 1.29 / 2.30 / 8.34,
+// key bundle 5.19 / 7.79 / 25.8 -> 2.46 / 4.49 / 16.5, plain 9.14 / 12.3 / 38.4 ->
+// 4.62 / 7.70 / 27.4.
 #pragma once
 
 #include "br_ntt.hpp"

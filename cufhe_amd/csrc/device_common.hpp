@@ -68,9 +68,7 @@ inline constexpr uint32_t kMaskRound = 1u << (32 - 2 - TP::nbit);
 // mantissa: adding 1.5 * 2^52 rounds at the unit position, so the low words
 // of the sum are the integer's. The Torus64 form takes 10 instructions; a
 // 64-bit integer conversion with its range test and mantissa shift took about
-// 40, which a lone lvl2 wave cannot hide (1000 lvl2 annihilations 466 -> 410 us,
-// one lvl02 MUX gate 21.7 -> 20.1 ms; the 2048-gate mix waits for its key
-// loads instead, 50.2 ms either way).
+// 40, which a lone lvl2 wave cannot hide (1000 lvl2 annihilations 466 -> 410 us).
 template <class T>
 __host__ __device__ __forceinline__ T double_to_torus(double v)
 {

@@ -89,10 +89,10 @@ __global__ __launch_bounds__(256) void k_from_fourier(double* out, const cplx* i
 
 // ---------------------------------------------------------------------------
 // Batched lvl2 rotation with two waves per job (CMUX keys; the key bundle with
-// two jobs per workgroup): C jobs per workgroup. The workgroups walk the job groups with a grid stride, so a grid that fits on
-// the device at once keeps every workgroup on the same rotation step: their
-// key reads then meet in L2 instead of drifting apart as later workgroups
-// start when earlier ones finish.
+// two jobs per workgroup): C jobs per workgroup. The workgroups walk the job
+// groups with a grid stride, so a grid that fits on the device at once keeps
+// every workgroup on the same rotation step: their key reads then meet in L2
+// instead of drifting apart as later workgroups start when earlier ones finish.
 template <bool KB, int C>
 __global__ __launch_bounds__(128 * C, C > 1 ? 1 : 3) void k_br_fft(const BrJob* __restrict__ jobs,
                                                                    int njobs, uint64_t mu,
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(512) void k_se_ks_lvl10(uint32_t* out, const uint32
 // help with the products and the roots (MUX/NMUX: two jobs of four transform
 // waves). Same key switch and rotation as the batched form, so the outputs are
 // the same words. One NAND of the lvl1 API took 3.80 ms with the rotation on a
-// single wave and the others only streaming the key; now 1.23 ms (MUX 4.40 ->
+// single wave and the others only streaming the key; now 1.25 ms (MUX 4.40 ->
 // 1.84 ms).
 template <bool KB, bool MUX>
 using GateShape = PwShape<lvl1param, MUX ? 2 : 1, 1, 8, MUX ? 0 : 4, KB>;
@@ -608,6 +608,11 @@ static void launch_br_lvl1(const BrJob* jobs, int njobs, int c, uint32_t mu,
 // CU; CMUX keys, or c = 2 (a tuning option, two jobs per workgroup): two waves
 // per job. All in a resident grid with a grid stride: the key (167 MB, bundle
 // 250 MB) outgrows the caches once the workgroups drift apart.
+// The bundle's workgroup fills a CU's LDS, so batches of several streams share
+// no CU as the two-wave workgroups did, two to a CU. Plans of 64 to 512 gates on
+// two to eight streams are up to 1.8 times as fast all the same; where all of
+// them together are just over a job per CU they need a second round, and three
+// streams of 96 or 128 gates or two of 192 take 10.8 ms (9.8 before).
 template <bool KB, int C>
 static void launch_br_two_wave(const BrJob* jobs, int njobs, uint64_t mu,
                                const FourierKeys<lvl2param>& K, hipStream_t st)

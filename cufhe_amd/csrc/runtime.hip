@@ -1323,7 +1323,7 @@ int cufhe_plan_create_lvl1(const cufhe_gate_desc* gates, int n, uint32_t* d_pool
     const int c = pick_c(jobs_per_group, s.k1.kb, nks);
     if (c < 0)
         return fail(CUFHE_ERR_UNSUPPORTED,
-                    "jobs_per_group must be 0, 1, 2, 4 or 8 (6: FFT key-bundle keys only)");
+                    "jobs_per_group must be 0, 1, 2, 4, 6 or 8 (6: not with FFT CMUX keys)");
     cufhe_plan* p = new cufhe_plan();
     p->c = c;
     p->use_graph = use_graph != 0;
@@ -1375,7 +1375,7 @@ int cufhe_plan_create_lvl01(const cufhe_gate_desc* gates, int n, uint32_t* d_poo
     const int c = pick_c(jobs_per_group, s.k1.kb, nbr);
     if (c < 0)
         return fail(CUFHE_ERR_UNSUPPORTED,
-                    "jobs_per_group must be 0, 1, 2, 4 or 8 (6: FFT key-bundle keys only)");
+                    "jobs_per_group must be 0, 1, 2, 4, 6 or 8 (6: not with FFT CMUX keys)");
     cufhe_plan* p = new cufhe_plan();
     p->level = 3;
     p->c = c;

@@ -184,11 +184,14 @@ int cufhe_gate_lvl02(int op, uint32_t* out, const uint32_t* in0, const uint32_t*
 
 /* Plan a batch of n gates over a device pool of lvl1 TLWEs (wire w at
  * d_pool + 1025 w). Outputs of a batch must not be read by the same batch.
- * jobs_per_group: bootstraps per workgroup (1, 2, 4, 6, 8; 0 = default).
- * With the FFT key-bundle keys, 6 and 8 (the default) mix workgroups of four,
- * two and one jobs by the size of the batch; with the NTT keys every value is
- * the same launch. use_graph != 0 captures the launches in a HIP graph
- * on the first run and replays it. */
+ * jobs_per_group: 1, 2, 4, 6, 8, or 0 for the autotuned value or the default
+ * (8); the outputs do not depend on it. With FFT key-bundle keys 1, 2 and 4 are
+ * the bootstraps of each workgroup, and 6 and 8 mix workgroups of four, two
+ * and one by the size of the batch. With FFT CMUX keys 1 and 2 are the
+ * bootstraps of each workgroup, 4 and 8 mix two and one, and 6 is refused.
+ * With NTT keys every value is the same launch, of up to eight a workgroup.
+ * use_graph != 0 captures the launches in a HIP graph on the first run and
+ * replays it. */
 int cufhe_plan_create_lvl1(const cufhe_gate_desc* gates, int n, uint32_t* d_pool,
                            int jobs_per_group, int use_graph, cufhe_plan** plan);
 /* Plan a batch of lvl02 gates (BR-IKS order) over a device pool of lvl0
@@ -204,7 +207,7 @@ int cufhe_plan_run(cufhe_plan* plan, void* stream);
 int cufhe_plan_destroy(cufhe_plan* plan);
 /* Bootstraps (blind rotations) a plan performs per run. */
 int cufhe_plan_bootstraps(const cufhe_plan* plan);
-/* Jobs per workgroup the plan launches with (after autotuning). */
+/* The jobs_per_group value the plan launches with (0 resolved). */
 int cufhe_plan_jobs_per_group(const cufhe_plan* plan);
 /* Run the plan eagerly with HIP events around each kernel on `stream`,
  * wait for it, and return the kernel durations in ms:

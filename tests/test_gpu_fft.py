@@ -396,11 +396,10 @@ def _run_gates_plain_pool(keys, ops, pool_ct, n):
 
 
 def test_shared_key_kernels_agree_at_scale(engine, keys_lvl1):
-    """2100 key-bundle gates (several rounds of workgroups, a partial last
-    workgroup for every kernel; 2100 jobs spread over 512 workgroups of 4 or
-    5): the one-job, the two-waves-per-job and the one-wave-per-job rotations
-    give identical ciphertexts, the default is the one-wave kernel, and every
-    gate decrypts right."""
+    """2100 key-bundle gates: one job per workgroup, and the mix (two full rounds
+    of four jobs per workgroup, the rest one by one; jobs_per_group 6, 8 and 0)
+    give identical ciphertexts, 0 is the default 8, and every gate decrypts
+    right."""
     load_lvl1(keys_lvl1, True)
     rng = np.random.default_rng(77)
     n = 2100
@@ -415,7 +414,6 @@ def test_shared_key_kernels_agree_at_scale(engine, keys_lvl1):
         dpool = C.DeviceBuffer.from_numpy(pool)
         plan = C.Plan(gates, dpool, jobs_per_group=c)
         if c == 0:
-            # key bundle: the one-wave-per-job kernel at every batch size
             assert plan.jobs_per_group == 8
         plan.run()
         C.check(C.lib().cufhe_synchronize(), "sync")
