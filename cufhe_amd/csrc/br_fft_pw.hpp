@@ -30,8 +30,8 @@
 // What bounds it: FP64 issue and LDS traffic, about equally, over the whole
 // CU. (An LDS KiB costs a CU 5.7 ns written and 3.2 ns read at two waves per
 // SIMD, a wave's FP64 instruction 0.5 ns; FP64 MFMA runs on the same pipe as
-// the vector FMAs.) At lvl2 phase 2 moves 786 KB of key a step at the 46
-// B/cycle that a CU's vector loads reach, and is bound by them.
+// the vector FMAs.) At lvl2 phase 2 also moves 786 KB of key a step through the
+// CU's vector loads, which reach about 46 B/cycle.
 #pragma once
 
 #include "br_fft.hpp"
@@ -304,10 +304,34 @@ struct PwWave {
         return v;
     }
 
+    // lvl2 batches: reads a word of every 128-byte line of a step's key, so that
+    // the key loads of that step find them in L2. `groups` workgroups, the first of
+    // the grid, rotate in step; those of an XCD (one in eight) share the lines over
+    // their four waves that are idle in phase 3. The key outgrows the caches next
+    // to the key-switching key, and a rotation that waits for it took 5.3 ms for 64
+    // to 256 jobs; 4.3 so (2048-gate mix 47.6 -> 42.1 ms). Fewer than 25 workgroups
+    // would need more than six loads a lane, which phase 3 does not hide (8 jobs
+    // 5.7 -> 7.5 ms), and read no lines ahead.
+    __device__ __forceinline__ void touch_key(int step, uint32_t groups) const
+    {
+        constexpr uint32_t kStep = S::NM * kTrgswFourier<P> * sizeof(cplx), kLine = 128;
+        const uint32_t waves = (groups + 7) / 8 * 4, mine = blockIdx.x / 8 * 4 + (qi - 2) * 2 + j;
+        if (waves * 64 * 6 * kLine < kStep) return;
+        const char* const p = reinterpret_cast<const char*>(K.bk) + static_cast<size_t>(step) * kStep;
+        uint32_t x = 0;
+#pragma unroll 6
+        for (uint32_t at = (mine * 64 + lane) * kLine; at < kStep; at += waves * 64 * kLine)
+            x ^= *reinterpret_cast<const uint32_t*>(p + at);
+        asm volatile("" ::"v"(x));
+    }
+
     // The rotation of the workgroup's jobs. mask: that of this wave's job, bar:
-    // its body's rotation. live: whether this wave's job exists. At the end the buffer of (job, j, digit 0) holds the N
-    // coefficients of component j (visible to the wave with qi = 0).
-    __device__ __forceinline__ void rotate(bool live, uint32_t bar, T mu, const PwMask& mask)
+    // its body's rotation. live: whether this wave's job exists. At the end the
+    // buffer of (job, j, digit 0) holds the N coefficients of component j (visible
+    // to the wave with qi = 0). TOUCH: touch_key ahead, with `groups`.
+    template <bool TOUCH = false>
+    __device__ __forceinline__ void rotate(bool live, uint32_t bar, T mu, const PwMask& mask,
+                                           uint32_t groups = 1)
     {
         constexpr int PF = S::PF, NB = S::NB;
         const int d0 = wave * S::BPL;
@@ -621,6 +645,8 @@ struct PwWave {
                     wave_lds_sync();
                 }
             }
+            if constexpr (TOUCH)
+                if (more && qi > 1) touch_key(next, groups);
             if (S::KB && live && rooter && more) {
                 put(roots);
                 if constexpr (S::kTail) tail_root = roots.v[0][0];

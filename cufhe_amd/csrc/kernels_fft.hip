@@ -173,7 +173,15 @@ __global__ __launch_bounds__(S::NT, WPE) void k_br_fft_pw(const BrJob* __restric
         const bool live = raw < njobs;
         const BrJob jb = jobs[live ? raw : njobs - 1];
         const PwMask mask{jb.in0, jb.in1, static_cast<uint32_t>(jb.ca), static_cast<uint32_t>(jb.cb)};
-        w.rotate(live, mask.body<P>(jb.offset), mu, mask);
+        if constexpr (S::kLvl1) {
+            w.rotate(live, mask.body<P>(jb.offset), mu, mask);
+        }
+        else {
+            // the workgroups that have a group in this round
+            const int left = ngroups - (grp - static_cast<int>(blockIdx.x));
+            w.template rotate<true>(live, mask.body<P>(jb.offset), mu, mask,
+                                    min(static_cast<int>(gridDim.x), left));
+        }
         if (live && w.qi == 0)
             pw_store<P>(reinterpret_cast<const T*>(w.buf(w.slot, w.j, 0)), w.j, w.lane,
                         jb.flags & kBrOutTrlwe, static_cast<T*>(jb.out));
@@ -609,10 +617,11 @@ static void launch_br_lvl1(const BrJob* jobs, int njobs, int c, uint32_t mu,
 // per job. All in a resident grid with a grid stride: the key (167 MB, bundle
 // 250 MB) outgrows the caches once the workgroups drift apart.
 // The bundle's workgroup fills a CU's LDS, so batches of several streams share
-// no CU as the two-wave workgroups did, two to a CU. Plans of 64 to 512 gates on
-// two to eight streams are up to 1.8 times as fast all the same; where all of
-// them together are just over a job per CU they need a second round, and three
-// streams of 96 or 128 gates or two of 192 take 10.8 ms (9.8 before).
+// no CU as the two-wave workgroups did, two to a CU. Plans of 1 to 900 gates on
+// two to eight streams are up to 2.2 times as fast all the same, but where all of
+// them together are up to a sixth over a job per CU: the few left then rotate in
+// a round of their own, with the key from memory (two streams of 130 gates 10.7
+// ms, of 150 10.0, of 200 9.5; 9.8 before).
 template <bool KB, int C>
 static void launch_br_two_wave(const BrJob* jobs, int njobs, uint64_t mu,
                                const FourierKeys<lvl2param>& K, hipStream_t st)

@@ -53,12 +53,14 @@ def test_widths_agree(rotations, c, n):
     assert np.array_equal(_run(tl0[:n], c), out[:n])
 
 
-def test_lvl2_bundle_equals_the_two_wave_kernel(keys_lvl2):
+# 25 workgroups are the fewest that read the key ahead; 259 leave three, and 300
+# leave 44 of 256 CUs for a second round
+@pytest.mark.parametrize("n", [24, 25, 259, 300])
+def test_lvl2_bundle_equals_the_two_wave_kernel(keys_lvl2, n):
     """Every bit: both forms do the same operations in the same order."""
     C.check(C.lib().cufhe_initialize(), "initialize")
     C.initialize_lvl02(keys_lvl2["bk_kb"], keys_lvl2["ksk"])
     rng = np.random.default_rng(62)
-    n = 259  # a job more than the CUs, and an odd one for the two-job groups
     tl0 = rng.integers(0, 2**32, (n, 637), dtype=np.uint64).astype(np.uint32)
     tl0[0] = 0
     tl0[1] = np.uint32(1 << 31)
